@@ -147,6 +147,9 @@ struct Context {
     // and apart from it, since the kernels of each step draw on ws.
     Workspace state;
     Tuning tune;
+    // The one-kernel Winograd conv's flag per workgroup (at most cu_count rounded up to
+    // eight), written and read by its launches on this stream alone.
+    int *wino_flags = nullptr;
     // GEMM launches timed on the device while tune.gemm_time is set: events
     // recorded before and after each launch (its split-K reduce included),
     // keyed by the kernel configuration, read and cleared by the caller.

@@ -191,6 +191,7 @@ Context::Context(int dev) : device(dev) {
     // The no-allocation entry points' fixed scratch: its device address on this GPU.
     noalloc_scratch_setup(dev);
     HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    dev_malloc(&wino_flags, size_t(cu_count + 8) * sizeof(int));
 }
 
 Context::~Context() {
@@ -200,6 +201,7 @@ Context::~Context() {
         (void)hipEventDestroy(g.stop);
     }
     for (hipEvent_t e : spare_events) (void)hipEventDestroy(e);
+    if (wino_flags) (void)hipFree(wino_flags);
     if (stream) (void)hipStreamDestroy(stream);
 }
 

@@ -198,27 +198,29 @@ void winograd_input_transform(Context &ctx, const float *x, int n, int h, int w,
 // m [16][tiles][c_out] -> out [n, H, W, c_out] = A^T m A + bias (+ residual2).
 void winograd_output_transform(Context &ctx, const float *m, int n, int h, int w, int c_out, bool upsample2x,
                                const float *bias, const float *residual2, float *out);
-// u [16][c_out][c_in] -> uf [16][c_in / 8][c_out][8], the fused kernel's operand order.
-void winograd_fused_weights(Context &ctx, const float *u, int c_out, int c_in, float *uf);
+// u [16][c_out][c_in] -> uf (winograd_fused_bytes), the fused kernel's operand: each
+// value split in three bf16 parts, in the order its waves read them.
+size_t winograd_fused_bytes(int c_out, int c_in);
+void winograd_fused_weights(Context &ctx, const float *u, int c_out, int c_in, void *uf);
 // Direct 3x3 conv, stride 1 / pad 1, for c_out <= 8 on maps of at least 65536
 // pixels (conv_small.hip), with the optional GN(+SiLU) prologue; false (nothing
 // launched) where it does not apply.
 bool conv3x3_small_co(Context &ctx, const float *x, int n, int h, int w, int c_in, const void *weight, WeightType wt,
                       int c_out, const float *bias, const Affine *prologue, float *out, const float *residual2);
 // The whole conv in one kernel (winograd_fused.hip) for f32 u, c_in % 32 == 0,
-// c_out % 64 == 0 and operands under 2 GiB; false (nothing launched) otherwise.
+// c_out % 64 == 0, the input under 1 GiB and u's copy under 2 GiB; false (nothing launched) otherwise.
 // uf: u in the fused order, or NULL (then made in the workspace for this call).
-// gn (optional): GroupNorm partials of out, blocks of 128 pixels (gn->rows set,
-// 0 where not written: odd output sizes, tiles per item not a multiple of 32).
+// gn (optional): GroupNorm partials of out, blocks of 256 pixels (gn->rows set,
+// 0 where not written: odd output sizes, tiles per item not a multiple of 64).
 bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, int c_in, const float *u,
-                            const float *uf, int c_out, const float *bias, bool upsample2x, const Affine *prologue,
+                            const void *uf, int c_out, const float *bias, bool upsample2x, const Affine *prologue,
                             float *out, const float *residual2, GnPartials *gn = nullptr);
 // The whole conv: u from winograd_weight_transform (ut kF32) or an f16 copy of it;
 // uf (optional) its fused-order copy for the one-kernel path; gn as above (only
 // the one-kernel path writes partials).
 void conv3x3_winograd(Context &ctx, const float *x, int n, int h, int w, int c_in, const void *u, WeightType ut,
                       int c_out, const float *bias, bool upsample2x, const Affine *prologue, float *out,
-                      const float *residual2 = nullptr, const float *uf = nullptr, GnPartials *gn = nullptr);
+                      const float *residual2 = nullptr, const void *uf = nullptr, GnPartials *gn = nullptr);
 void selftest_mfma_f32(Context &ctx, const float *a_host, const float *b_host, float *d_host);
 
 // ---- lambda layers (lambda.hip), src/unet/lambda.rs

@@ -123,14 +123,14 @@ const void *WeightStore::winograd_kernel_f16(const float *u, int co, int ci) con
     return u16;
 }
 
-const float *WeightStore::winograd_kernel_fused(const float *u, int co, int ci) const {
-    const size_t bytes = size_t(16) * co * ci * sizeof(float);
+const void *WeightStore::winograd_kernel_fused(const float *u, int co, int ci) const {
+    const size_t bytes = winograd_fused_bytes(co, ci);
     void *uf = nullptr;
     mh::dev_malloc(&uf, bytes);
     derived_.push_back(uf);
     derived_bytes_ += bytes;
-    winograd_fused_weights(ctx_, u, co, ci, static_cast<float *>(uf));
-    return static_cast<const float *>(uf);
+    winograd_fused_weights(ctx_, u, co, ci, uf);
+    return uf;
 }
 
 DParam WeightStore::get(const std::string &name, int64_t numel, bool gemm) const {

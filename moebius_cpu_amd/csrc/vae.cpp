@@ -87,7 +87,7 @@ struct Conv3v {
     bool up = false;
     DParam w;
     const float *u = nullptr;
-    const float *uf = nullptr;  // u in the one-kernel path's order (channel counts it takes)
+    const void *uf = nullptr;  // u in the one-kernel path's order (channel counts it takes)
     const float *b = nullptr;
     void load(const WeightStore &W, const std::string &p, int ci_, int co_, int stride_ = 1,
               const int *pad_ = nullptr, bool up_ = false) {

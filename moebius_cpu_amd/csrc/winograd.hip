@@ -239,7 +239,7 @@ void winograd_output_transform(Context &ctx, const float *m, int n, int h, int w
 
 void conv3x3_winograd(Context &ctx, const float *x, int n, int h, int w, int c_in, const void *u, WeightType ut,
                       int c_out, const float *bias, bool upsample2x, const Affine *prologue, float *out,
-                      const float *residual2, const float *uf, GnPartials *gn) {
+                      const float *residual2, const void *uf, GnPartials *gn) {
     if (gn) gn->rows = 0;
     MH_REQUIRE(c_in > 0 && c_out > 0 && c_in % 4 == 0 && c_out % 4 == 0,
                "Winograd conv: channel counts must be multiples of 4");

@@ -1,38 +1,40 @@
 // Winograd F(2x2, 3x3) conv in one kernel (src/engine/winograd.rs:48-120):
 // the input transform, the 16 plane products and the output transform of a
-// block of 32 tiles x 64 output channels stay on chip, so V and M (16 planes
+// block of 64 tiles x 64 output channels stay on chip, so V and M (16 planes
 // of tiles x channels each) never reach HBM. The separate path writes and
 // reads both: about 4.2 GB per 512x512x128 conv of the VAE decoder.
 //
-// Workgroup: 512 threads, one per CU (LDS: two V stages of 72 KB), walking
-// a share of the (channel block, tile block) items. Per chunk of 32 input
-// channels every thread transforms one tile's 4x4 patch for two channels (the
-// reference's operation order, as wino_input_kernel) into the V stage
-// [plane][tile][channel]; the 16 channel pairs of a tile sit on adjacent
-// lanes, so a patch load reads 128-byte runs. Wave w (of 8, two per SIMD)
-// multiplies planes 2w and 2w + 1 on v_mfma_f32_32x32x2f32 (tiles x 64
-// channels, two 32x32 blocks per plane), reading V from LDS and U from global
-// memory (L2 resident) in the fused order [16][ci / 8][co][8]: the 32
-// channels of one block at one K sub-step are 1 KB of consecutive bytes, so
-// each U load of a wave reads whole cache lines (from [16][co][ci] a load
-// touches 32 lines for 32 bytes each). The next chunk's patch loads are in
-// flight during the current chunk's last three quarters of products. At the
-// end the 16 planes go through LDS and each thread applies the output
-// transform (winograd.rs:329-352, as wino_output_kernel) to one tile and four
-// channels, adding bias and the optional residual.
+// Workgroup: 512 threads, one per CU (LDS: two V stages of 64 KB), walking a
+// share of the (channel block, tile block) items. Per chunk of 16 input channels
+// every thread transforms one tile's 4x4 patch for two channels (the reference's
+// operation order, as wino_input_kernel) into the V stage [plane][tile][channel];
+// the 8 channel pairs of a tile sit on adjacent lanes, so a patch load reads
+// 64-byte runs. Wave w (of 8, two per SIMD) multiplies planes 2w and 2w + 1 on
+// v_mfma_f32_32x32x16_bf16 with both operands split in three bf16 parts
+// (split_bf16.hpp): V from LDS in f32, split by the one wave that reads it, U from
+// global memory (L2 resident) split at load and packed so that every load of a wave
+// is one run of 1 KB. At the end the planes go through LDS, half the tiles at a
+// time, and each thread applies the output transform (winograd.rs:329-352, as
+// wino_output_kernel) to one tile and four channels, adding bias and the optional
+// residual.
 //
-// At 512x512x128 -> 128 (A/B on MI355X): 730 us for transforms + batched
-// GEMM; this kernel with U in [16][co][ci] order and a tile's channels on
-// lanes 32 apart, 495 us (with its MFMAs removed it still took 490 us: the
-// operand loads bound it); with the layouts above 372 us; one workgroup per
-// CU with the next item's loads issued early, 361 us; every thread a
-// producer, 358 us (256x256x256: 347 -> 334, upsampled 128x128x512:
-// 1327 -> 1286). The products alone run at 91% of the f32 MFMA peak.
+// What bounds it (MI355X, 512x512x128 -> 128, parts taken out of a copy): the
+// products alone 130 us, with the transforms 148, with the patch and U loads 221,
+// with the output transform and its stores 279; on the f32 instructions the same
+// conv took 358 us, its products alone 239. The loads cost what they do because
+// the vector L1 serves 96 KB of U and 64 KB of patches per chunk and workgroup:
+// 64 tiles per workgroup, twice what the f32 kernel took, halve U's share, and
+// 128 accumulators per lane are what that leaves room for. The registers are full:
+// a few more live values spill the patch in the loop (392 us), so the output
+// transform's numbers are derived anew from the thread's, the patch's validity is
+// kept in scalar masks and the next item's loads wait for the sums to leave.
+// 128x128x512 -> 512: 402 us in f32, 251 here. VAE decode 12.97 -> 9.77 ms.
 #include <algorithm>
 
 #include "common.hpp"
 #include "dmath.hpp"
 #include "kernels.hpp"
+#include "split_bf16.hpp"
 
 namespace mh {
 namespace {
@@ -41,33 +43,36 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-constexpr int kFT = 32;        // tiles per workgroup
+constexpr int kFT = 64;        // tiles per workgroup
 constexpr int kFC = 64;        // output channels per workgroup
-constexpr int kFK = 32;        // input channels per chunk
-constexpr int kVS = kFK + 4;   // V row stride in LDS (floats)
-constexpr int kMS = kFC + 4;   // M row stride in LDS (floats)
-constexpr int kVStage = 16 * kFT * kVS;
-constexpr int kLds = 2 * kVStage;  // 36864 floats = 144 KB
-static_assert(16 * kFT * kMS <= kLds, "the M exchange fits in the V stages");
-constexpr int kRed = 16 * kFT * kMS;  // GroupNorm reduction scratch, past the M exchange
-static_assert(kRed + 2 * 8 * 64 <= kLds && kRed >= kVStage, "reduction scratch fits, in V stage 1");
-constexpr int kOob = int(0x80000000u);
+constexpr int kFK = 16;        // input channels per chunk: one matrix instruction's K
+constexpr int kVStage = 16 * kFT * kFK;  // floats; 16-byte quads of a row swizzled (vquad)
+constexpr int kHT = kFT / 2;             // tiles per half of the M exchange
+constexpr int kMS = kFC + 4;             // M row stride in LDS (floats)
+constexpr int kRed = 16 * kHT * kMS;     // GroupNorm reduction scratch, past the M exchange
+constexpr int kLds = kRed + 2 * 8 * 64;  // floats, 140 KB
+static_assert(2 * kVStage <= kLds && kRed >= kVStage, "the V stages fit, the scratch in stage 1 or past it");
+constexpr int kOob = int(0x80000000u);   // past any buffer: reads zero
+constexpr int kUBlk = 1024;              // bytes of one packed U block: 32 channels x 16 K of one part
 
 struct FGeo {
     int h, w, hi, wi, th, tw;
-    int64_t tiles;
+    int tiles;  // the input's 1 GiB holds fewer than 2^23 pixels
+};
+
+struct FArgs {
+    const float *x;
+    const char *u;  // packed (wino_u_fused_kernel)
+    const float *psc, *psh, *bias, *res2;
+    float *out, *gnp;
+    int *sick;  // per workgroup: whether it met a sum that is infinite or NaN
+    FGeo g;
+    uint32_t x_bytes, u_bytes;
+    int ci, co, psilu, nco_blocks, nwork;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), short(0), int(bytes), 0x00020000);
-}
-
-__device__ __forceinline__ floatx4 ld4(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-
-__device__ __forceinline__ floatx2 ld2(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
 
 __device__ __forceinline__ floatx4 sub4(floatx4 a, floatx4 b) { return floatx4{a[0] - b[0], a[1] - b[1], a[2] - b[2], a[3] - b[3]}; }
@@ -76,16 +81,18 @@ __device__ __forceinline__ floatx4 add4(floatx4 a, floatx4 b) { return floatx4{a
 constexpr int kFThreads = 512;  // 8 waves, two per SIMD
 constexpr int kFPlanes = 16 / (kFThreads / 64);  // planes per wave
 
+// Where quad q (4 channels) of tile row t sits in its 64-byte V row: rows four
+// apart take different banks.
+__device__ __forceinline__ int vquad(int t, int q) { return (q ^ ((t >> 2) & 3)) * 4; }
+
 template <int UP, bool PRO>
-__global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(const float *__restrict__ x, uint32_t x_bytes, FGeo g,
-                                                            int ci, const float *__restrict__ u, uint32_t u_bytes,
-                                                            int co, const float *__restrict__ psc,
-                                                            const float *__restrict__ psh, int psilu,
-                                                            const float *__restrict__ bias,
-                                                            const float *__restrict__ res2, float *__restrict__ out,
-                                                            float *__restrict__ gnp, int nco_blocks, int nwork) {
-    __shared__ float lds[kLds];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
+    const FGeo &g = a.g;
+    const int ci = a.ci, co = a.co, nwork = a.nwork;
+    __shared__ __align__(16) float lds[kLds];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const SplitSel sel = split_sel();
     // Work items (channel block, tile block), channel block outer. Workgroup i
     // runs on XCD i % 8 (round-robin dispatch); each XCD takes one contiguous
     // eighth of the items, so it works through few channel blocks and their U
@@ -93,79 +100,77 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(const float *_
     // of that range. The grid holds one workgroup per CU, and a workgroup
     // issues its next item's first patch and U loads before the current
     // item's last products and output transform, which hide their latency.
-    const int ntb = nwork / nco_blocks;
+    const int ntb = nwork / a.nco_blocks;
     const int per_xcd = (nwork + 7) / 8;
     const int slots = int(gridDim.x) / 8;
     const int item_end = min(nwork, (int(blockIdx.x) % 8 + 1) * per_xcd);
-    int item = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
-    if (item >= item_end) return;
-    const __amdgpu_buffer_rsrc_t xr = rsrc(x, x_bytes), ur = rsrc(u, u_bytes);
+    const int first = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
+    if (first >= item_end) {
+        if (tid == 0) a.sick[blockIdx.x] = 0;
+        return;
+    }
+    const __amdgpu_buffer_rsrc_t ur = rsrc(a.u, a.u_bytes);
     const int per_item = g.th * g.tw;
-    const int n_items = int(g.tiles / per_item);
+    const int n_items = g.tiles / per_item;
 
-    // Producer role (every thread, so the transform's work is spread over
-    // both waves of each SIMD): tile vt of the block, channel pair vq of the
-    // chunk; the 16 pairs of a tile sit on 16 adjacent lanes (128-byte runs).
-    const int vq = tid & (kFK / 2 - 1), vt = (tid >> 4) & (kFT - 1);
-    // Consumer role: wave w, planes kFPlanes w .. + kFPlanes - 1, two 32x32 blocks of 64 channels.
-    // Lane l reads a float4 along K of row l % 32 at K offset 4 (l / 32); MFMA t
-    // takes its component t, so both operands pair k = 8 s + 4 (l / 32) + t.
-    const int row = lane & 31, kq = 4 * (lane >> 5);
-    // Per item: the block's first tile and channel; the producer's patch
-    // origin (byte offset of source pixel (sy - 1, sx - 1), channel 4 vq; the
-    // patch's rows and columns sit at -1, 0, 1, 2 from (sy, sx), or -1, 0, 0, 1
-    // when upsampling) with one bit per pixel inside the image, and its batch
-    // item; the consumer's U offsets in [16][ci / 8][co][8] (plane
-    // kFPlanes w + p, channel co0 + 32 j + row, K offset kq within the
-    // sub-step's 8; sub-step k8 adds k8 * co * 8 floats).
-    int64_t t0 = 0;
-    int co0 = 0, vb = 0, porg = 0;
-    unsigned valid = 0;
-    int uoff[kFPlanes][2];
+    // Producer role (every thread): tile vt of the block, channel pair vq of the
+    // chunk; the 8 pairs of a tile sit on 8 adjacent lanes (64-byte runs).
+    const int vq = tid & (kFK / 2 - 1), vt = tid >> 3;
+    // Consumer role: wave w, planes kFPlanes w .. + kFPlanes - 1, two 32-tile by two
+    // 32-channel blocks. Lane l holds row l % 32, K 8 (l / 32) .. + 7 of the chunk.
+    const int row = lane & 31, kg = lane >> 5;
+    // Per item: the block's first tile and channel; the producer's source pixel, which
+    // of its patch's rows and columns (at -1, 0, 1, 2 from it, at -1, 0, 0, 1 when
+    // upsampling) are inside the image, and its batch item; the wave's first U block
+    // (kUBlk bytes each, plane-major [plane][ci / 16][co / 32][part]).
+    int t0 = 0, co0 = 0, vb = 0, ubase = 0;
+    int porg = 0;                   // bytes of source pixel (sy, sx), channel 2 vq; the buffer starts a row and a
+    bool rowin[4], colin[4];        // pixel early, so that a patch row or column's step is never negative
     const int prow = g.w * ci * 4, pcol = ci * 4;  // bytes per source row, per pixel
     constexpr int kStep[4] = {0, 1, 2 - UP, 3 - UP};  // patch row / column k -> source offset + 1
-    auto setup = [&](int it) {
-        t0 = int64_t(it % ntb) * kFT;
-        co0 = (it / ntb) * kFC;
-        const int64_t tv = t0 + vt;
-        const int b = int(tv / per_item), rem = int(tv - int64_t(b) * per_item);
+    const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char *>(a.x) - prow - pcol, a.x_bytes + prow + pcol);
+    auto setup_producer = [&](int it) {
+        int ptid = tid;
+        asm volatile("" : "+v"(ptid));
+        const int tv = it % ntb * kFT + (ptid >> 3);
+        const int b = tv / per_item, rem = tv - b * per_item;
         const int ty = rem / g.tw, tx = rem - ty * g.tw;
         vb = min(b, n_items - 1);  // a tile past the end reads nothing, but keeps its prologue loads in range
         const int sy = (2 * ty) >> UP, sx = (2 * tx) >> UP;
-        porg = tv < g.tiles ? (((b * g.h + sy - 1) * g.w + sx - 1) * ci + 2 * vq) * 4 : 0;
-        valid = 0;
+        porg = ((b * g.h + sy) * g.w + sx) * pcol + 8 * (ptid & (kFK / 2 - 1));
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            const int iy = 2 * ty + (kk >> 2) - 1, ix = 2 * tx + (kk & 3) - 1;
-            const bool in = tv < g.tiles && iy >= 0 && iy < g.hi && ix >= 0 && ix < g.wi;
-            valid |= in ? (1u << kk) : 0u;
+        for (int k = 0; k < 4; ++k) {
+            const int iy = 2 * ty + k - 1, ix = 2 * tx + k - 1;
+            rowin[k] = tv < g.tiles && iy >= 0 && iy < g.hi;
+            colin[k] = ix >= 0 && ix < g.wi;
         }
-#pragma unroll
-        for (int p = 0; p < kFPlanes; ++p)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                uoff[p][j] = ((((kFPlanes * wave + p) * (ci / 8)) * co + co0 + 32 * j + row) * 8 + kq) * 4;
+    };
+    auto setup_consumer = [&](int it) {
+        t0 = it % ntb * kFT;
+        co0 = (it / ntb) * kFC;
+        ubase = ((kFPlanes * wave * (ci / kFK)) * (co / 32) + co0 / 32) * 3 * kUBlk;
     };
     floatx2 d[16];
     auto produce = [&](int kc) {
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            const int off = porg + kStep[kk >> 2] * prow + kStep[kk & 3] * pcol + kc * kFK * 4;
-            d[kk] = ld2(xr, (valid >> kk) & 1u ? off : kOob);
-        }
+        for (int kk = 0; kk < 16; ++kk)
+            d[kk] = __builtin_bit_cast(
+                floatx2, __builtin_amdgcn_raw_buffer_load_b64(
+                             xr, rowin[kk >> 2] && colin[kk & 3] ? porg : kOob,
+                             kStep[kk >> 2] * prow + kStep[kk & 3] * pcol + kc * kFK * 4, 0));
     };
     auto transform_store = [&](int kc, int stage) {
         if constexpr (PRO) {
             const int c = kc * kFK + 2 * vq;
-            const floatx2 sc = *reinterpret_cast<const floatx2 *>(psc + int64_t(vb) * ci + c);
-            const floatx2 sh = *reinterpret_cast<const floatx2 *>(psh + int64_t(vb) * ci + c);
+            const floatx2 sc = *reinterpret_cast<const floatx2 *>(a.psc + int64_t(vb) * ci + c);
+            const floatx2 sh = *reinterpret_cast<const floatx2 *>(a.psh + int64_t(vb) * ci + c);
 #pragma unroll
             for (int kk = 0; kk < 16; ++kk) {
-                if (valid & (1u << kk)) {
+                if (rowin[kk >> 2] && colin[kk & 3]) {
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         float y = __builtin_fmaf(d[kk][e], sc[e], sh[e]);
-                        if (psilu) y = ref_silu(y);
+                        if (a.psilu) y = ref_silu(y);
                         d[kk][e] = y;
                     }
                 }
@@ -180,147 +185,178 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(const float *_
             tt[8 + col] = d2 - d1;
             tt[12 + col] = d1 - d3;
         }
-        float *vs = lds + stage * kVStage + vt * kVS + 2 * vq;
+        float *vs = lds + stage * kVStage + vt * kFK + vquad(vt, vq >> 1) + 2 * (vq & 1);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const floatx2 *q = tt + r * 4;
-            *reinterpret_cast<floatx2 *>(vs + (r * 4) * kFT * kVS) = q[0] - q[2];
-            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 1) * kFT * kVS) = q[1] + q[2];
-            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 2) * kFT * kVS) = q[2] - q[1];
-            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 3) * kFT * kVS) = q[1] - q[3];
+            *reinterpret_cast<floatx2 *>(vs + (r * 4) * kFT * kFK) = q[0] - q[2];
+            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 1) * kFT * kFK) = q[1] + q[2];
+            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 2) * kFT * kFK) = q[2] - q[1];
+            *reinterpret_cast<floatx2 *>(vs + (r * 4 + 3) * kFT * kFK) = q[1] - q[3];
         }
     };
 
-    floatx16 acc[kFPlanes][2];
-    // Loads are waited for in issue order, so the order is chosen to never
-    // wait on more than the next operands: U for sub-step 1 is issued with
-    // sub-step 0, U for sub-steps 2 and 3 with sub-step 1 and after them the
-    // next chunk's patch (it lands during the last three sub-steps' products;
-    // the transform waits for it), and U for the next chunk's first sub-step
-    // after the last products, to land during the transform.
-    static_assert(kFK / 8 == 4, "four K sub-steps per chunk");
-    floatx4 b0[kFPlanes][2], b1[kFPlanes][2], b2[kFPlanes][2], b3[kFPlanes][2];
-    auto load_b = [&](floatx4 (&dst)[kFPlanes][2], int kc, int s) {
+    floatx16 acc[kFPlanes][2][2];  // [plane][tile block][channel block]
+    static_assert(kFPlanes == 2, "two planes per wave, taken in turn");
+    // U parts of plane p, chunk kc: six whole blocks.
+    auto load_u = [&](int p, int kc, bf16x8 (&dst)[2][3]) {
+        const int off = ubase + ((p * (ci / kFK) + kc) * (co / 32)) * 3 * kUBlk;
 #pragma unroll
-        for (int p = 0; p < kFPlanes; ++p)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) dst[p][j] = ld4(ur, uoff[p][j] + (kc * (kFK / 8) + s) * co * 32);
+            for (int q = 0; q < 3; ++q)
+                dst[j][q] = __builtin_bit_cast(
+                    bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ur, lane * 16, off + (j * 3 + q) * kUBlk, 0));
     };
-    auto mfma_step = [&](const float *vs, int s, const floatx4 (&b)[kFPlanes][2]) {
-        floatx4 a[kFPlanes];
+    const int vlo = (kFPlanes * wave * kFT + row) * kFK + vquad(row, 2 * kg);
+    const int vhi = (kFPlanes * wave * kFT + row) * kFK + vquad(row, 2 * kg + 1);
+    // V rows of plane p, tile block i from LDS, split.
+    auto read_v = [&](const float *vs, int p, int i, Split3 &v) {
+        // rows 32 apart share their swizzle
+        const floatx4 lo = *reinterpret_cast<const floatx4 *>(vs + vlo + (p * kFT + 32 * i) * kFK);
+        const floatx4 hi = *reinterpret_cast<const floatx4 *>(vs + vhi + (p * kFT + 32 * i) * kFK);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            split_pair(e < 2 ? lo[2 * e] : hi[2 * e - 4], e < 2 ? lo[2 * e + 1] : hi[2 * e - 3], e, sel, v);
+    };
+    auto products = [&](int p, int i, const Split3 &v, const bf16x8 (&uu)[2][3]) {
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[p][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v.q[kSplitTerm[t][0]].v,
+                                                                      uu[j][kSplitTerm[t][1]], acc[p][i][j], 0, 0, 0);
+    };
+    const int nk = ci / kFK;
+    float sick = 0.0f;  // NaN once any sum is infinite or NaN
+    int item = first;
+    setup_producer(item);
+    setup_consumer(item);
+    bf16x8 u0[2][3], u1[2][3];
+    produce(0);
+    load_u(0, 0, u0);
+    for (;;) {
+        const int next = item + slots;
+        const bool has_next = next < item_end;
+        transform_store(0, 0);
+        produce(1);
 #pragma unroll
         for (int p = 0; p < kFPlanes; ++p)
-            a[p] = *reinterpret_cast<const floatx4 *>(vs + (kFPlanes * wave + p) * kFT * kVS + 8 * s);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[p][i][j][v] = 0.f;
+        __syncthreads();
+        // Four steps of twelve products per chunk, each with the split of the next
+        // step's V between them, the last with the next chunk's transform. The loads
+        // are spread over the chunk and waited for in issue order: the patch of the
+        // chunk after next once the transform has used its registers, the second
+        // plane's U at the start of the chunk, the next chunk's first U half way.
+        for (int kc = 0; kc < nk; ++kc) {
+            const float *vs = lds + (kc & 1) * kVStage;
+            load_u(1, kc, u1);
+            __builtin_amdgcn_sched_barrier(0);
+            Split3 v;
+            read_v(vs, 0, 0, v);
+            products(0, 0, v, u0);
+            __builtin_amdgcn_sched_barrier(0);
+            read_v(vs, 0, 1, v);
+            products(0, 1, v, u0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_u(0, min(kc + 1, nk - 1), u0);
+            read_v(vs, 1, 0, v);
+            products(1, 0, v, u1);
+            __builtin_amdgcn_sched_barrier(0);
+            read_v(vs, 1, 1, v);
+            products(1, 1, v, u1);
+            if (kc + 1 < nk) transform_store(kc + 1, (kc + 1) & 1);
+            if (kc + 2 < nk) produce(kc + 2);
+            __syncthreads();
+        }
+        const int et0 = t0, eco0 = co0;
+        // the thread's number again, so that nothing the output transform derives from
+        // it is kept in registers through the products
+        int etid = tid;
+        asm volatile("" : "+v"(etid));
+        const int elane = etid & 63;
+        float *const mw = lds + (kFPlanes * wave * kHT + 4 * (elane >> 5)) * kMS + (elane & 31);
+#pragma unroll
+        for (int p = 0; p < kFPlanes; ++p)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sick = __builtin_fmaf(acc[p][i][j][v], 0.0f, sick);
+
+        floatx4 gs{0.f, 0.f, 0.f, 0.f}, gq = gs;  // GroupNorm sums of the values stored
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            // M [16][tile][channel] of 32 tiles through LDS: register v of lane l holds
+            // row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of its block.
+            if (half) __syncthreads();  // the first half's reads are done
 #pragma unroll
             for (int p = 0; p < kFPlanes; ++p)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    acc[p][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[p][t], b[p][j][t], acc[p][j], 0, 0, 0);
-    };
-    const int nk = ci / kFK;
-    setup(item);
-    produce(0);
-    load_b(b0, 0, 0);
-    for (;;) {
-        transform_store(0, 0);
 #pragma unroll
-        for (int p = 0; p < kFPlanes; ++p)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[p][j][v] = 0.f;
-        __syncthreads();
-        const int next = item + slots;
-        const bool has_next = next < item_end;
-        const int64_t et0 = t0;
-        const int eco0 = co0;
-        for (int kc = 0; kc < nk; ++kc) {
-            const bool more = kc + 1 < nk;
-            const float *vs = lds + (kc & 1) * kVStage + row * kVS + kq;
-            load_b(b1, kc, 1);
-            mfma_step(vs, 0, b0);
-            load_b(b2, kc, 2);
-            load_b(b3, kc, 3);
-            if (more) {
-                produce(kc + 1);
-            } else if (has_next) {  // this item's U loads are all issued: switch to the next
-                setup(next);
+                    for (int v = 0; v < 16; ++v)
+                        mw[(p * kHT + 8 * (v >> 2) + (v & 3)) * kMS + 32 * j] = acc[p][half][j][v];
+            if (half) {  // the sums have left their registers: the next item's first loads (the last item's
+                         // again at the end, so that nothing older stays live)
+                setup_consumer(has_next ? next : item);
+                setup_producer(has_next ? next : item);
+                load_u(0, 0, u0);
                 produce(0);
             }
-            mfma_step(vs, 1, b1);
-            mfma_step(vs, 2, b2);
-            mfma_step(vs, 3, b3);
-            if (more) {
-                load_b(b0, kc + 1, 0);
-                transform_store(kc + 1, (kc + 1) & 1);
-            } else if (has_next) {
-                load_b(b0, 0, 0);
-            }
             __syncthreads();
-        }
-
-    // M [16][tile][channel] through LDS: register v of lane l holds row
-    // 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of its block.
+            const int tl = etid >> 4, q = etid & 15;
+            const int t = et0 + kHT * half + tl;
+            if (t >= g.tiles) continue;
+            const int b = t / per_item, rem = t - b * per_item;
+            const int ty = rem / g.tw, tx = rem - ty * g.tw;
+            const float *src = lds + tl * kMS + 4 * q;
+            floatx4 m0[4], m1[4];
 #pragma unroll
-    for (int p = 0; p < kFPlanes; ++p)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int tr = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                lds[((kFPlanes * wave + p) * kFT + tr) * kMS + 32 * j + row] = acc[p][j][v];
+            for (int rr = 0; rr < 4; ++rr) {
+                const floatx4 aa = *reinterpret_cast<const floatx4 *>(src + (rr * 4) * kHT * kMS);
+                const floatx4 bb = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 1) * kHT * kMS);
+                const floatx4 cc = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 2) * kHT * kMS);
+                const floatx4 dd = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 3) * kHT * kMS);
+                m0[rr] = add4(add4(aa, bb), cc);
+                m1[rr] = sub4(sub4(bb, cc), dd);
+                asm volatile("" ::: "memory");  // sixteen rows at once would not fit the registers
             }
-    __syncthreads();
+            const int c = eco0 + 4 * q;
+            const floatx4 bv = a.bias ? *reinterpret_cast<const floatx4 *>(a.bias + c) : floatx4{0.f, 0.f, 0.f, 0.f};
+            floatx4 y[4];
+            y[0] = add4(add4(add4(m0[0], m0[1]), m0[2]), bv);
+            y[1] = add4(add4(add4(m1[0], m1[1]), m1[2]), bv);
+            y[2] = add4(sub4(sub4(m0[1], m0[2]), m0[3]), bv);
+            y[3] = add4(sub4(sub4(m1[1], m1[2]), m1[3]), bv);
 #pragma unroll
-    for (int r = 0; r < (kFT * kFC / 4) / kFThreads; ++r) {
-        const int item = tid + kFThreads * r;
-        const int tl = item / (kFC / 4), q = item - tl * (kFC / 4);
-        const int64_t t = et0 + tl;
-        if (t >= g.tiles) continue;
-        const int b = int(t / per_item), rem = int(t - int64_t(b) * per_item);
-        const int ty = rem / g.tw, tx = rem - ty * g.tw;
-        const float *src = lds + tl * kMS + 4 * q;
-        floatx4 u0[4], u1[4];
+            for (int kk = 0; kk < 4; ++kk) {
+                const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
+                if (oy >= g.hi || ox >= g.wi) continue;
+                const int64_t o = int64_t((b * g.hi + oy) * g.wi + ox) * co + c;
+                floatx4 rv = y[kk];
+                if (a.res2) rv = add4(rv, *reinterpret_cast<const floatx4 *>(a.res2 + o));
+                *reinterpret_cast<floatx4 *>(a.out + o) = rv;
+                if (a.gnp) {
+                    gs = add4(gs, rv);
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const floatx4 a = *reinterpret_cast<const floatx4 *>(src + (rr * 4) * kFT * kMS);
-            const floatx4 bb = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 1) * kFT * kMS);
-            const floatx4 cc = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 2) * kFT * kMS);
-            const floatx4 dd = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 3) * kFT * kMS);
-            u0[rr] = add4(add4(a, bb), cc);
-            u1[rr] = sub4(sub4(bb, cc), dd);
-        }
-        const int c = eco0 + 4 * q;
-        const floatx4 bv = bias ? *reinterpret_cast<const floatx4 *>(bias + c) : floatx4{0.f, 0.f, 0.f, 0.f};
-        floatx4 gs{0.f, 0.f, 0.f, 0.f}, gq = gs;  // GroupNorm sums of the values stored
-        floatx4 y[4];
-        y[0] = add4(add4(add4(u0[0], u0[1]), u0[2]), bv);
-        y[1] = add4(add4(add4(u1[0], u1[1]), u1[2]), bv);
-        y[2] = add4(sub4(sub4(u0[1], u0[2]), u0[3]), bv);
-        y[3] = add4(sub4(sub4(u1[1], u1[2]), u1[3]), bv);
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
-            if (oy >= g.hi || ox >= g.wi) continue;
-            const int64_t o = ((int64_t(b) * g.hi + oy) * g.wi + ox) * co + c;
-            floatx4 rv = y[kk];
-            if (res2) rv = add4(rv, *reinterpret_cast<const floatx4 *>(res2 + o));
-            *reinterpret_cast<floatx4 *>(out + o) = rv;
-            if (gnp) {
-                gs = add4(gs, rv);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) gq[e] = __builtin_fmaf(rv[e], rv[e], gq[e]);
+                    for (int e = 0; e < 4; ++e) gq[e] = __builtin_fmaf(rv[e], rv[e], gq[e]);
+                }
             }
         }
-        if (gnp) {
+        if (a.gnp) {
             // GroupNorm partials of this block (per channel: sum and sum of
-            // squares over its 128 pixels), for the next GroupNorm's fold in
+            // squares over its 256 pixels), for the next GroupNorm's fold in
             // place of a statistics pass: the four threads of a wave that hold
-            // channel quad q (tiles 4w .. 4w + 3) by xor butterfly, then the
-            // eight waves in order through LDS past the M exchange (V stage 1,
-            // not written again before the next item's second chunk).
+            // channel quad q (tiles 4w .. 4w + 3 of each half) by xor butterfly,
+            // then the eight waves in order through LDS past the M exchange.
 #pragma unroll
             for (int off = 16; off < 64; off <<= 1)
 #pragma unroll
@@ -329,72 +365,174 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(const float *_
                     gq[e] += __shfl_xor(gq[e], off, 64);
                 }
             floatx4 *red = reinterpret_cast<floatx4 *>(lds + kRed);
-            if (lane < kFC / 4) {
-                red[wave * (kFC / 4) + lane] = gs;
-                red[(kFThreads / 64 + wave) * (kFC / 4) + lane] = gq;
+            if (elane < kFC / 4) {
+                red[wave * (kFC / 4) + elane] = gs;
+                red[(kFThreads / 64 + wave) * (kFC / 4) + elane] = gq;
             }
             __syncthreads();
-            if (tid < kFC / 4) {
-                floatx4 ts = red[tid], tq = red[(kFThreads / 64) * (kFC / 4) + tid];
+            if (etid < kFC / 4) {
+                floatx4 ts = red[etid], tq = red[(kFThreads / 64) * (kFC / 4) + etid];
 #pragma unroll
                 for (int w8 = 1; w8 < kFThreads / 64; ++w8) {
-                    ts = add4(ts, red[w8 * (kFC / 4) + tid]);
-                    tq = add4(tq, red[(kFThreads / 64 + w8) * (kFC / 4) + tid]);
+                    ts = add4(ts, red[w8 * (kFC / 4) + etid]);
+                    tq = add4(tq, red[(kFThreads / 64 + w8) * (kFC / 4) + etid]);
                 }
-                float *dst = gnp + ((et0 / kFT) * co + eco0 + 4 * tid) * 2;
+                float *dst = a.gnp + (int64_t(et0 / kFT) * co + eco0 + 4 * etid) * 2;
                 *reinterpret_cast<floatx4 *>(dst) = floatx4{ts[0], tq[0], ts[1], tq[1]};
                 *reinterpret_cast<floatx4 *>(dst + 4) = floatx4{ts[2], tq[2], ts[3], tq[3]};
             }
         }
-    }
         if (!has_next) break;
         __syncthreads();  // the output transform's reads of M are done before V stage 0 is written
         item = next;
     }
+    const int bad = __syncthreads_or(sick != sick);
+    if (tid == 0) a.sick[blockIdx.x] = bad;
 }
 
-// u [16][co][ci] -> uf [16][ci / 8][co][8], one float4 per thread.
-__global__ void wino_u_fused_kernel(const float *__restrict__ u, int co, int ci, float *__restrict__ uf) {
-    const int64_t total4 = int64_t(16) * co * ci / 4;
-    for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < total4; e += int64_t(gridDim.x) * blockDim.x) {
-        const int64_t f = e * 4, plane_sz = int64_t(co) * ci;
-        const int64_t plane = f / plane_sz, rem = f - plane * plane_sz;
-        const int k8 = int(rem / (int64_t(co) * 8));
-        const int r2 = int(rem - int64_t(k8) * co * 8), c = r2 >> 3, kk = r2 & 7;
-        *reinterpret_cast<floatx4 *>(uf + f) =
-            *reinterpret_cast<const floatx4 *>(u + (plane * co + c) * ci + k8 * 8 + kk);
+// The outputs of one work item that are infinite or NaN, again in f32 on the vector
+// unit: a part product of an infinite value with a zero part is NaN where the f32
+// product is infinite, and a value within half a bf16 step of the largest f32
+// rounds to an infinite part. A kernel of its own, launched after each conv and done
+// at once where no workgroup flagged its sums (in the conv kernel's tail the same code
+// cost it registers: 353 against 274 us at 512x512x128 -> 128).
+__device__ __forceinline__ void wino_mend(const FArgs &a, int up, bool pro, int t0, int co0) {
+    const FGeo &g = a.g;
+    const int per_item = g.th * g.tw, ci = a.ci, co = a.co;
+#pragma nounroll
+    for (int e = threadIdx.x; e < kFT * kFC * 4; e += blockDim.x) {
+        const int t = t0 + e / (kFC * 4);
+        const int o = co0 + e % kFC, kk = (e / kFC) % 4;
+        if (t >= g.tiles) continue;
+        const int b = t / per_item, rem = t - b * per_item;
+        const int ty = rem / g.tw, tx = rem - ty * g.tw;
+        const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
+        if (oy >= g.hi || ox >= g.wi) continue;
+        const int64_t oi = ((int64_t(b) * g.hi + oy) * g.wi + ox) * co + o;
+        if (__builtin_fabsf(a.out[oi]) < __builtin_inff()) continue;
+        // A^T m A: nine planes with their signs, row by row, in the transform's order
+        float y = 0.0f, line = 0.0f;
+#pragma nounroll
+        for (int n = 0; n < 9; ++n) {
+            const int r = n / 3 + (kk >> 1), c4 = n % 3 + (kk & 1);
+            float m = 0.0f;
+#pragma nounroll
+            for (int c = 0; c < ci; ++c) {
+                float v = 0.0f, col = 0.0f;
+#pragma nounroll
+                for (int q = 0; q < 4; ++q) {
+                    // V of plane (r, c4): rows pr and columns pc of the patch with their signs
+                    const int qr = q & 1, qc = q >> 1;
+                    const int pr = r == 0 ? 2 * qr : r == 1 ? 1 + qr : r == 2 ? 2 - qr : 1 + 2 * qr;
+                    const int pc = c4 == 0 ? 2 * qc : c4 == 1 ? 1 + qc : c4 == 2 ? 2 - qc : 1 + 2 * qc;
+                    const int iy = 2 * ty + pr - 1, ix = 2 * tx + pc - 1;
+                    float dv = 0.0f;
+                    if (iy >= 0 && iy < g.hi && ix >= 0 && ix < g.wi) {
+                        dv = a.x[((int64_t(b) * g.h + (iy >> up)) * g.w + (ix >> up)) * ci + c];
+                        if (pro) {
+                            dv = __builtin_fmaf(dv, a.psc[int64_t(b) * ci + c], a.psh[int64_t(b) * ci + c]);
+                            if (a.psilu) dv = ref_silu(dv);
+                        }
+                    }
+                    col = !qr ? dv : r == 1 ? col + dv : col - dv;
+                    if (qr) v = !qc ? col : c4 == 1 ? v + col : v - col;
+                }
+                const char *blk = a.u + ((int64_t(4 * r + c4) * (ci / kFK) + c / kFK) * (co / 32) + o / 32) * 3 * kUBlk +
+                                  (((o % 32) + 32 * ((c % kFK) / 8)) * 8 + c % 8) * 2;
+                float uv = float(*reinterpret_cast<const __bf16 *>(blk + 2 * kUBlk));
+                uv = float(*reinterpret_cast<const __bf16 *>(blk + kUBlk)) + uv;
+                uv = float(*reinterpret_cast<const __bf16 *>(blk)) + uv;
+                m = __builtin_fmaf(v, uv, m);
+            }
+            line = n % 3 == 0 ? m : (kk & 1) ? line - m : line + m;
+            if (n % 3 == 2) y = n == 2 ? line : (kk >> 1) ? y - line : y + line;
+        }
+        if (a.bias) y = y + a.bias[o];
+        if (a.res2) y = y + a.res2[oi];
+        a.out[oi] = y;
+    }
+}
+
+// One workgroup per workgroup of the conv, over its items.
+__global__ __launch_bounds__(kFThreads) void wino_mend_kernel(FArgs a, int up, int pro) {
+    if (!a.sick[blockIdx.x]) return;
+    const int per_xcd = (a.nwork + 7) / 8, ntb = a.nwork / a.nco_blocks;
+    const int end = min(a.nwork, (int(blockIdx.x) % 8 + 1) * per_xcd);
+    for (int it = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8; it < end; it += int(gridDim.x) / 8)
+        wino_mend(a, up, pro != 0, it % ntb * kFT, it / ntb * kFC);
+}
+
+// u [16][co][ci] -> packed [16][ci / 16][co / 32][part][lane][8]: lane l of a block
+// holds channel l % 32, K 8 (l / 32) .. + 7. An infinite or NaN value keeps itself
+// in the first part alone, and one that rounds to infinity is cut off instead.
+__global__ void wino_u_fused_kernel(const float *__restrict__ u, int co, int ci, char *__restrict__ uf) {
+    const SplitSel sel = split_sel();
+    const int64_t blocks = int64_t(16) * (ci / kFK) * (co / 32);
+    for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < blocks * 64;
+         e += int64_t(gridDim.x) * blockDim.x) {
+        const int lane = int(e & 63);
+        const int64_t blk = e >> 6;
+        const int cb = int(blk % (co / 32));
+        const int64_t r = blk / (co / 32);
+        const int kc = int(r % (ci / kFK)), plane = int(r / (ci / kFK));
+        const float *src = u + (int64_t(plane) * co + cb * 32 + (lane & 31)) * ci + kc * kFK + 8 * (lane >> 5);
+        Split3 s;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const float a = src[2 * p], b = src[2 * p + 1];
+            split_pair(a, b, p, sel, s);
+            const float v[2] = {a, b};
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (__builtin_fabsf(static_cast<float>(s.q[0].p[p][h])) < __builtin_inff()) continue;
+                if (__builtin_fabsf(v[h]) < __builtin_inff()) {
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, v[h]);
+                    const float hi = __builtin_bit_cast(float, bits & 0xffff0000u), rest = v[h] - hi;
+                    s.q[0].p[p][h] = static_cast<__bf16>(hi);
+                    s.q[1].p[p][h] = static_cast<__bf16>(rest);
+                    s.q[2].p[p][h] = static_cast<__bf16>(rest - static_cast<float>(s.q[1].p[p][h]));
+                } else {
+                    s.q[0].p[p][h] = static_cast<__bf16>(v[h]);
+                    s.q[1].p[p][h] = s.q[2].p[p][h] = static_cast<__bf16>(0.0f);
+                }
+            }
+        }
+        char *dst = uf + blk * 3 * kUBlk + lane * 16;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8 *>(dst + q * kUBlk) = s.q[q].v;
     }
 }
 
 template <int UP, bool PRO>
-void launch_fused(Context &ctx, int nwork, const float *x, uint32_t xb, const FGeo &g, int ci, const float *u,
-                  uint32_t ub, int co, const Affine *pro, const float *bias, const float *res2, float *out,
-                  float *gnp) {
+void launch_fused(Context &ctx, const FArgs &a) {
     // one workgroup per CU (its LDS holds one), a multiple of 8 (see the work
     // order in the kernel), no more than the items of one XCD's share need
-    const int64_t per_xcd = ceil_div(nwork, 8);
+    const int64_t per_xcd = ceil_div(a.nwork, 8);
     const unsigned grid = unsigned(8 * std::max<int64_t>(1, std::min<int64_t>(ctx.cu_count / 8, per_xcd)));
-    wino_fused_kernel<UP, PRO><<<grid, kFThreads, 0, ctx.stream>>>(x, xb, g, ci, u, ub, co, pro ? pro->scale : nullptr,
-                                                             pro ? pro->shift : nullptr, pro && pro->silu ? 1 : 0,
-                                                             bias, res2, out, gnp, co / kFC, nwork);
+    wino_fused_kernel<UP, PRO><<<grid, kFThreads, 0, ctx.stream>>>(a);
+    MH_LAUNCH_CHECK();
+    wino_mend_kernel<<<grid, kFThreads, 0, ctx.stream>>>(a, UP, PRO);
 }
 
 }  // namespace
 
-void winograd_fused_weights(Context &ctx, const float *u, int c_out, int c_in, float *uf) {
-    MH_REQUIRE(c_in % 8 == 0 && aligned16(u) && aligned16(uf), "Winograd fused weights: c_in % 8, 16-byte aligned");
-    const int64_t total4 = int64_t(16) * c_out * c_in / 4;
-    if (total4 == 0) return;
-    const unsigned blocks = unsigned(std::min<int64_t>(ceil_div(total4, 256), 65536));
-    wino_u_fused_kernel<<<blocks, 256, 0, ctx.stream>>>(u, c_out, c_in, uf);
+size_t winograd_fused_bytes(int c_out, int c_in) { return size_t(16) * c_out * c_in * 6; }
+
+void winograd_fused_weights(Context &ctx, const float *u, int c_out, int c_in, void *uf) {
+    MH_REQUIRE(c_in % kFK == 0 && c_out % 32 == 0 && aligned16(u) && aligned16(uf),
+               "Winograd fused weights: c_in % 16, c_out % 32, 16-byte aligned");
+    const int64_t lanes = int64_t(16) * (c_in / kFK) * (c_out / 32) * 64;
+    if (lanes == 0) return;
+    const unsigned blocks = unsigned(std::min<int64_t>(ceil_div(lanes, 256), 65536));
+    wino_u_fused_kernel<<<blocks, 256, 0, ctx.stream>>>(u, c_out, c_in, static_cast<char *>(uf));
     MH_LAUNCH_CHECK();
 }
 
 bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, int c_in, const float *u,
-                            const float *uf, int c_out, const float *bias, bool upsample2x, const Affine *prologue,
+                            const void *uf, int c_out, const float *bias, bool upsample2x, const Affine *prologue,
                             float *out, const float *residual2, GnPartials *gn) {
     if (gn) gn->rows = 0;
-    if (ctx.tune.wino_fused == 0 || c_in % kFK || c_out % kFC) return false;
+    if (ctx.tune.wino_fused == 0 || c_in % 32 || c_out % kFC) return false;
     // Where it is faster (A/B per conv on MI355X, three kernels -> this one):
     // 512x512x128 746 -> 419 us, 256x256x256 552 -> 401, the same upsampled
     // 1824 -> 1352, 128x128x512 437 -> 402, the same upsampled 1471 -> 1335;
@@ -405,41 +543,46 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
     if (ctx.tune.wino_fused < 0 && (c_in > 512 || c_out > 512)) return false;
     if (!aligned16(x) || !aligned16(u) || !aligned16(out) || !aligned16(bias) || !aligned16(residual2)) return false;
     if (prologue && (!aligned16(prologue->scale) || !aligned16(prologue->shift))) return false;
-    const int64_t x_bytes = int64_t(n) * h * w * c_in * 4, u_bytes = int64_t(16) * c_out * c_in * 4;
-    if (x_bytes >= (int64_t(1) << 31) || u_bytes >= (int64_t(1) << 31)) return false;
+    const int64_t x_bytes = int64_t(n) * h * w * c_in * 4, u_bytes = int64_t(winograd_fused_bytes(c_out, c_in));
+    if (x_bytes >= (int64_t(1) << 30) || u_bytes >= (int64_t(1) << 31)) return false;
     FGeo g;
     const int up = upsample2x ? 1 : 0;
     g.h = h, g.w = w, g.hi = h << up, g.wi = w << up;
     g.th = (g.hi + 1) / 2, g.tw = (g.wi + 1) / 2;
-    g.tiles = int64_t(n) * g.th * g.tw;
-    if (ctx.tune.wino_fused < 0 && g.tiles < 4096) return false;
-    if (g.tiles == 0) return true;
-    const int64_t blocks = ceil_div(g.tiles, kFT) * (c_out / kFC);
+    const int64_t tiles = int64_t(n) * g.th * g.tw;
+    if (ctx.tune.wino_fused < 0 && tiles < 4096) return false;
+    if (tiles == 0) return true;
+    g.tiles = int(tiles);
+    const int64_t blocks = ceil_div(tiles, kFT) * (c_out / kFC);
     if (blocks >= (int64_t(1) << 30)) return false;
     const int nwork = int(blocks);
     const uint32_t xb = uint32_t(x_bytes), ub = uint32_t(u_bytes);
     if (!uf) {  // no precomputed fused-order copy: make one in the workspace
-        float *tmp = static_cast<float *>(ctx.ws.get(size_t(u_bytes), ctx.stream));
+        void *tmp = ctx.ws.get(size_t(u_bytes), ctx.stream);
         winograd_fused_weights(ctx, u, c_out, c_in, tmp);
         uf = tmp;
     } else if (!aligned16(uf)) {
         return false;
     }
-    u = uf;
-    // GroupNorm partials: blocks of 32 whole tiles (128 pixels) within one item
+    // GroupNorm partials: blocks of 64 whole tiles (256 pixels) within one item
     float *gnp = nullptr;
     if (gn && gn->part && aligned16(gn->part) && g.hi % 2 == 0 && g.wi % 2 == 0 &&
         int64_t(g.th) * g.tw % kFT == 0 && gn->item_rows == g.hi * g.wi) {
         gnp = gn->part;
         gn->rows = 4 * kFT;
     }
-    if (up) {
-        if (prologue) launch_fused<1, true>(ctx, nwork, x, xb, g, c_in, u, ub, c_out, prologue, bias, residual2, out, gnp);
-        else launch_fused<1, false>(ctx, nwork, x, xb, g, c_in, u, ub, c_out, prologue, bias, residual2, out, gnp);
-    } else {
-        if (prologue) launch_fused<0, true>(ctx, nwork, x, xb, g, c_in, u, ub, c_out, prologue, bias, residual2, out, gnp);
-        else launch_fused<0, false>(ctx, nwork, x, xb, g, c_in, u, ub, c_out, prologue, bias, residual2, out, gnp);
-    }
+    const FArgs a{x,    static_cast<const char *>(uf),
+                  prologue ? prologue->scale : nullptr,
+                  prologue ? prologue->shift : nullptr,
+                  bias, residual2,
+                  out,  gnp,
+                  ctx.wino_flags,
+                  g,    xb,
+                  ub,   c_in,
+                  c_out, prologue && prologue->silu ? 1 : 0,
+                  c_out / kFC, nwork};
+    if (up) prologue ? launch_fused<1, true>(ctx, a) : launch_fused<1, false>(ctx, a);
+    else prologue ? launch_fused<0, true>(ctx, a) : launch_fused<0, false>(ctx, a);
     MH_LAUNCH_CHECK();
     return true;
 }
