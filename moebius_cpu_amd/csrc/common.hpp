@@ -56,7 +56,8 @@ struct ShapePlan {
 // (MOEBIUS_HIP_GEMM_PLAN, _GN_IN_MAXC, _DW_TILED, _TAP_HEADS, _CROSS_HEADS,
 // _GN_BLOCKS, _GN_APPLY, _WINO_FUSED, _UP_CONCAT, _LAMBDA_TAPS, _GEMM_LOG,
 // _GEMM_WIDE, _LN_FOLD, _TAP_SPLIT, _GEMM_TIME, _TAPS_ROWS, _CROSS_MFMA, _TAP_SLICE,
-// _TAP_JQ, _TAP_FUSED, _GEMM_SHAPE_PLAN, _TAPS_R16, _WINO_U16, _WINO_V16, _DW_OUT16)
+// _TAP_JQ, _TAP_FUSED, _GEMM_SHAPE_PLAN, _TAPS_R16, _WINO_U16, _WINO_V16, _DW_OUT16,
+// _GEMM_SPLIT)
 // when a context is created and changed with set_tuning (mh_context_set_tuning).
 // The defaults are the measured choices; nothing on the hot path reads the
 // environment.
@@ -94,6 +95,9 @@ struct Tuning {
                            // bit 0 k = 40 (the 64x64 latents), bit 1 k = 80, bit 2 k = 160
     int taps_r16 = 0;      // FAST contexts: 1 the self-lambda position products on f16-rounded operands
                            // (as the FAST GEMMs take them); 0 on the f32 operands (faster)
+    int gemm_split = 1;    // EXACT GEMMs on the bf16 matrix instructions with f32 operands split in three (0: the f32
+                           // instructions); "tm,bn,wm,wk" forces its tiling
+    int split_tm = 0, split_bn = 0, split_wm = 0, split_wk = 0;
     int wino_u16 = 1;      // FAST contexts: the UNet's Winograd plane GEMMs read U stored in f16 (0: f32,
                            // rounded on every load; the same products)
     int wino_v16 = 1;      // FAST contexts with an f16 U: the input transform writes V in f16 (0: f32)

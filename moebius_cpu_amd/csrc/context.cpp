@@ -119,6 +119,16 @@ bool set_tuning(Tuning &t, const char *key, const char *value) {
     if (k == "taps_r16") return to_int(t.taps_r16, 0) && t.taps_r16 >= 0 && t.taps_r16 <= 1;
     if (k == "wino_u16") return to_int(t.wino_u16, 1) && t.wino_u16 >= 0 && t.wino_u16 <= 1;
     if (k == "wino_v16") return to_int(t.wino_v16, 1) && t.wino_v16 >= 0 && t.wino_v16 <= 1;
+    if (k == "gemm_split") {  // "0", "1" or "tm,bn,wm,wk"
+        t.split_tm = t.split_bn = t.split_wm = t.split_wk = 0;
+        t.gemm_split = 1;
+        int tm = 0, bn = 0, wm = 0, wk = 0;
+        if (std::sscanf(v.c_str(), "%d,%d,%d,%d", &tm, &bn, &wm, &wk) == 4) {
+            t.split_tm = tm, t.split_bn = bn, t.split_wm = wm, t.split_wk = wk;
+            return true;
+        }
+        return to_int(t.gemm_split, 1) && t.gemm_split >= 0 && t.gemm_split <= 1;
+    }
     if (k == "dw_out16") return to_int(t.dw_out16, 1) && t.dw_out16 >= 0 && t.dw_out16 <= 1;
     if (k == "tap_jq") return to_int(t.tap_jq, 1) && (t.tap_jq == 1 || t.tap_jq == 2);
     if (k == "tap_slice") return to_int(t.tap_slice, 0) && t.tap_slice >= 0 && t.tap_slice <= 64;
@@ -172,6 +182,7 @@ Context::Context(int dev) : device(dev) {
                                               {"MOEBIUS_HIP_WINO_U16", "wino_u16"},
                                               {"MOEBIUS_HIP_WINO_V16", "wino_v16"},
                                               {"MOEBIUS_HIP_DW_OUT16", "dw_out16"},
+                                              {"MOEBIUS_HIP_GEMM_SPLIT", "gemm_split"},
                                               {"MOEBIUS_HIP_LN_FOLD", "ln_fold"},
                                               {"MOEBIUS_HIP_TAP_SPLIT", "tap_split"}};
     for (const auto &kv : env_keys)

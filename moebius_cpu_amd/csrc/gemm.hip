@@ -1,4 +1,7 @@
-// GEMM-shaped convolutions on gfx950 matrix cores (f32 MFMA, f32 accumulate).
+// GEMM-shaped convolutions on gfx950 matrix cores, f32 accumulate: EXACT products
+// on the bf16 instructions with each f32 operand split in three (gemm_split.hpp), or
+// on the f32 instructions where those are faster (plan_split) and for operands that
+// have no 16-byte quads; FAST ones in f16 (gemm_h16.hpp).
 //
 //   1x1 conv  (src/engine/conv.rs:38-55):  out[P x Co] = x[P x Ci] . W[Co x Ci]^T
 //   3x3 conv  (src/engine/conv.rs:83-165): implicit GEMM, M = output pixels,
@@ -9,7 +12,7 @@
 //             GroupNorm affine (+SiLU) prologue of src/engine/norm.rs:33-37.
 //
 // Both operands are K-contiguous (NHWC activations; [Co][.. Ci] weights), so
-// one "NT" kernel serves every shape. Tiles: BM x BN x 32 per 256-thread
+// one "NT" kernel serves every shape. The f32 kernel's tiles: BM x BN x 32 per 256-thread
 // workgroup, four 64-wide waves in a 2x2 arrangement, each owning
 // (BM/2) x (BN/2) of the output as 32x32 blocks of v_mfma_f32_32x32x2f32.
 // Each lane reads a float4 along K from LDS for A and for B and issues four
@@ -23,6 +26,7 @@
 // tiles are summed in a fixed order by a reduction kernel that also applies
 // bias / residual / SiLU, so results are deterministic run to run.
 #include "gemm_h16.hpp"
+#include "gemm_split.hpp"
 
 namespace mh {
 using namespace gemm;
@@ -35,16 +39,16 @@ uint32_t extent(int64_t rows, int64_t ld, int64_t cols, int esz) {
     return uint32_t(bytes);
 }
 
-// Context precision selects the kernel family: EXACT runs f32 matrix
-// instructions, FAST the f16 ones (activations rounded to f16 as they load).
+// Context precision selects the kernel family: EXACT runs the split bf16 or f32
+// matrix instructions, FAST the f16 ones (activations rounded to f16 as they load).
 void run_dense(Context &ctx, GemmArgs &p, WeightType wt, GemmEpilogue epi, int batch, bool vec) {
     if (ctx.precision == Precision::Fast) launch_dense_h16(ctx, p, wt, epi, batch, vec);
-    else launch_dense(ctx, p, wt, epi, batch, vec);
+    else if (!vec || !launch_split_dense(ctx, p, wt, epi, batch)) launch_dense(ctx, p, wt, epi, batch, vec);
 }
 
 void run_conv(Context &ctx, GemmArgs &p, WeightType wt, int mode, bool pro) {
     if (ctx.precision == Precision::Fast) launch_conv_h16(ctx, p, wt, mode, pro);
-    else launch_conv(ctx, p, wt, mode, pro);
+    else if (!launch_split_conv(ctx, p, wt, mode, pro)) launch_conv(ctx, p, wt, mode, pro);
 }
 
 __global__ void im2col_gather_kernel(GemmArgs p, int64_t first, int64_t count, float *__restrict__ rows) {
@@ -140,7 +144,7 @@ void conv1x1(Context &ctx, const float *x, int64_t pixels, int c_in, const void 
         p.psilu = x_aff->silu ? 1 : 0;
         p.pro_rows = x_aff->rows_per_item;
         if (ctx.precision == Precision::Fast) launch_dense_pro_h16(ctx, p, wt, epi);
-        else launch_dense_pro(ctx, p, wt, epi);
+        else if (!launch_split_dense_pro(ctx, p, wt, epi)) launch_dense_pro(ctx, p, wt, epi);
     } else if (c_in % 4 == 0 && aligned16(x)) {
         run_dense(ctx, p, wt, epi, 1, true);
     } else {
@@ -226,7 +230,7 @@ void conv1x1_ln(Context &ctx, const float *x, int64_t pixels, int c_in, const Ln
         p.b = f.w32;
         p.ln_c1 = f.c1_32;
         p.b_bytes = extent(n, c_in, c_in, 4);
-        launch_dense_ln(ctx, p, kF32, epi);
+        if (!launch_split_dense_ln(ctx, p, kF32, epi)) launch_dense_ln(ctx, p, kF32, epi);
     }
 }
 

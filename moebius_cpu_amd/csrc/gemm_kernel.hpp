@@ -675,12 +675,13 @@ __device__ __forceinline__ void ln_stats_from_parts(const GemmArgs &p, int m0, f
 // a (BM / WM) x (BN / WN) block of it, times WK wave groups that split every
 // LDS stage's K between them (their sums are added in group order in the
 // epilogue). 2x2x1 is the original layout of the square tiles.
-template <int BM, int BN, int WM, int WN, int WK>
+// MFO: the matrix block size where it is not the f32 kernel's choice (0).
+template <int BM, int BN, int WM, int WN, int WK, int MFO = 0>
 struct Waves {
     static constexpr int kWaves = WM * WN * WK;
     static constexpr int kThreads = 64 * kWaves;
     static constexpr int TM = BM / WM, TN = BN / WN;
-    static constexpr int MF = (TM % 32 == 0 && TN % 32 == 0) ? 32 : 16;
+    static constexpr int MF = MFO ? MFO : ((TM % 32 == 0 && TN % 32 == 0) ? 32 : 16);
     static constexpr int FM = TM / MF, FN = TN / MF;
     static constexpr int CS = BN + (MF == 16 ? 4 : 8);  // C tile row stride (floats)
     // The 2x2 layout's epilogue, where each thread keeps one column quad over its
@@ -697,19 +698,37 @@ struct Waves {
     }
 };
 
+struct NoMend {
+    __device__ void operator()(float *) const {}
+};
+
+// Four columns of the C tile's WK partial sums (SLAB floats apart), in group order.
+template <int WK, int SLAB>
+__device__ __forceinline__ float4 sum_groups(const float *c) {
+    float4 t = *reinterpret_cast<const float4 *>(c);
+#pragma unroll
+    for (int w = 1; w < WK; ++w) {
+        const float4 u = *reinterpret_cast<const float4 *>(c + w * SLAB);
+        t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
+    }
+    return t;
+}
+
 // Epilogue through LDS, shared by the f32 and f16 kernels (smem holds at least
 // WK * BM * CS floats, plus 2048 floats or, outside the 2x2 layout, BM * CS +
 // 8 * NT for the GroupNorm sums, and is free): block (i, j), register v, lane l
 // of wave (wm, wn, wk) holds row acc_row(v, l), column l % MF of its group's
 // partial sum; the K groups' tiles are added in LDS, then each thread finishes
 // four adjacent columns of a row at a time (16-byte loads and stores), or one
-// element at a time where that is not possible.
+// element at a time where that is not possible. mend (optional): called with the
+// whole C tile where any thread passes bad, before it is finished.
 template <int BM, int BN, int WM, int WN, int WK, int MF, int EPI, bool SPLIT, bool FSILU = false,
-          bool OUT16 = false, typename Acc, int FM, int FN>
+          bool OUT16 = false, typename Acc, int FM, int FN, typename Mend = NoMend>
 __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const Acc (&acc)[FM][FN], int m0, int n0,
-                                           int z, const float *ln_st = nullptr) {
+                                           int z, const float *ln_st = nullptr, bool bad = false,
+                                           const Mend &mend = Mend()) {
     using MI = Mf<MF>;
-    using L = Waves<BM, BN, WM, WN, WK>;
+    using L = Waves<BM, BN, WM, WN, WK, MF>;
     constexpr int NT = L::kThreads;
     // C tile row stride: the lane groups of one register's store sit 4 rows
     // apart (16x16 blocks: 16 columns per group) or 4 rows apart in two halves
@@ -730,20 +749,27 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const
                 for (int v = 0; v < MI::kAccRegs; ++v)
                     slab[(r0 + i * MF + MI::acc_row(v, lane)) * CS + c0 + j * MF] = acc[i][j][v];
     }
-    __syncthreads();
-    if constexpr (WK > 1) {  // K groups' partial tiles summed in group order into the first
-        constexpr int C4 = BN / 4;
-        for (int e = tid; e < BM * C4; e += NT) {
-            const int rr = e / C4, cc = (e - rr * C4) * 4;
-            float4 t = *reinterpret_cast<const float4 *>(smem + rr * CS + cc);
-#pragma unroll
-            for (int w = 1; w < WK; ++w) {
-                const float4 u = *reinterpret_cast<const float4 *>(smem + w * BM * CS + rr * CS + cc);
-                t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
+    int any_bad = 0;
+    if constexpr (std::is_same_v<Mend, NoMend>) __syncthreads();
+    else any_bad = __syncthreads_or(bad);
+    // K groups' partial tiles: summed in group order as the store pass reads them, or
+    // here into the first where the tile is needed whole.
+    const bool summed = WK == 1 || p.vec_out != 1 || any_bad;
+    if constexpr (WK > 1) {
+        if (summed) {
+            constexpr int C4 = BN / 4;
+            for (int e = tid; e < BM * C4; e += NT) {
+                const int rr = e / C4, cc = (e - rr * C4) * 4;
+                *reinterpret_cast<float4 *>(smem + rr * CS + cc) = sum_groups<WK, BM * CS>(smem + rr * CS + cc);
             }
-            *reinterpret_cast<float4 *>(smem + rr * CS + cc) = t;
+            __syncthreads();
         }
-        __syncthreads();
+    }
+    if constexpr (!std::is_same_v<Mend, NoMend>) {
+        if (any_bad) {
+            mend(smem);
+            __syncthreads();
+        }
     }
     if (p.vec_out == 1) {
         constexpr int C4 = BN / 4;  // float4 per tile row
@@ -787,7 +813,7 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const
                 const int row = m0 + rr, col = n0 + cc;
                 if (row >= p.M || col >= p.N) continue;
                 float *c = smem + rr * CS + cc;
-                float4 v = *reinterpret_cast<const float4 *>(c);
+                float4 v = summed ? *reinterpret_cast<const float4 *>(c) : sum_groups<WK, BM * CS>(c);
                 if (ln_st) v = ln_correct(p, ln_st, rr, col, v);
                 if (SPLIT) {
                     *reinterpret_cast<float4 *>(p.partial + (int64_t(z) * p.M + row) * p.N + col) = v;

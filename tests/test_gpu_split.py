@@ -9,6 +9,8 @@ import pytest
 
 import oracle
 from moebius_cpu_amd import engine as E
+from moebius_cpu_amd import unet_params as U
+from moebius_cpu_amd.unet import UNet
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +77,83 @@ def test_winograd_error_and_odd_values(ctx, n, h, w, ci, co, up):
     x = odd_values(x)
     assert same_kind(run(x, 1), oracle.conv3x3(x, wt, b, upsample2x=up))
     assert same_kind(run(np.full_like(x, np.nan), 1), np.full(want.shape, np.nan))
+
+
+# every tiling of the split GEMM (csrc/gemm_split.hpp) and the planner's choice
+TILES = ["1", "16,80,8,1", "16,64,8,1", "16,80,4,2", "16,64,4,2", "16,48,4,2", "16,80,2,4", "16,64,2,4", "16,48,2,4",
+         "16,32,2,4"]
+
+
+def gemm_bound(k):
+    """A chain of k / 32 f32 sums, each rounded once (2^-24 in 2-norm at most), the
+    sum of the small part products and the epilogue's two additions."""
+    return 2.0 ** -24 * (4 + np.sqrt(k / 32))
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("f16", [False, True])
+# one row, one K step; rows, columns and K past their last whole tile, stage and quad
+@pytest.mark.parametrize("h,w,ci,co", [(1, 1, 4, 4), (9, 11, 200, 70), (33, 3, 36, 324), (16, 16, 1284, 96)])
+def test_gemm_tilings(ctx, tune, tile, f16, h, w, ci, co):
+    rng = np.random.default_rng(h + ci + co)
+    x = rng.standard_normal((2, h, w, ci)).astype(np.float32)
+    wt = (rng.standard_normal((co, ci)) / np.sqrt(ci)).astype(np.float16 if f16 else np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    r = rng.standard_normal((2, h, w, co)).astype(np.float32)
+    param = E.Param(ctx, wt, f16=f16)
+
+    def run(x, tile):
+        tune("gemm_split", tile)
+        out = E.Tensor(ctx)
+        E.Conv1x1(ctx, ci, co, param, b).forward(E.Tensor.from_numpy(ctx, x), out, E.Tensor.from_numpy(ctx, r))
+        return out.numpy()
+
+    print(f"split gemm {tile} 2x{h}x{w} {ci}->{co} f16={f16}", flush=True)
+    want = x.astype(np.float64) @ wt.T.astype(np.float64) + b + r
+    assert rel(run(x, tile), want) <= gemm_bound(ci)
+    if h > 3 and w > 4:
+        x = odd_values(x)
+        assert same_kind(run(x, tile), run(x, "0"))
+
+
+@pytest.mark.parametrize("tile", TILES)
+# the gathers: 64 channels to a K step and 4, stride 2, the upsample; a GroupNorm prologue
+@pytest.mark.parametrize("h,w,ci,co,stride,up,pro", [(13, 9, 64, 80, 1, False, False), (15, 11, 36, 52, 2, False, False),
+                                                     (7, 5, 64, 40, 1, True, True), (6, 9, 20, 33, 1, False, True)])
+def test_conv_tilings(ctx, tune, tile, h, w, ci, co, stride, up, pro):
+    rng = np.random.default_rng(h + ci + co)
+    x = rng.standard_normal((2, h, w, ci)).astype(np.float32)
+    wt = (rng.standard_normal((co, 3, 3, ci)) / np.sqrt(9 * ci)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    aff, xs = None, x.astype(np.float64)
+    if pro:
+        sc = (1 + 0.2 * rng.standard_normal((2, ci))).astype(np.float32)
+        sh = rng.standard_normal((2, ci)).astype(np.float32)
+        aff = E.Affine(E.DeviceArray.from_numpy(ctx, sc), E.DeviceArray.from_numpy(ctx, sh), False)
+        xs = xs * sc.reshape(2, 1, 1, ci) + sh.reshape(2, 1, 1, ci)
+    if up:
+        xs = xs.repeat(2, axis=1).repeat(2, axis=2)
+    xp = np.pad(xs, ((0, 0), (1, 1), (1, 1), (0, 0)))
+    oh, ow = -(-xs.shape[1] // stride), -(-xs.shape[2] // stride)
+    want = b + sum(xp[:, ky:ky + stride * oh:stride, kx:kx + stride * ow:stride][:, :oh, :ow]
+                   @ wt[:, ky, kx].T.astype(np.float64) for ky in range(3) for kx in range(3))
+    print(f"split conv {tile} 2x{h}x{w} {ci}->{co} stride={stride} up={up} pro={pro}", flush=True)
+    tune("gemm_split", tile)
+    out = E.Tensor(ctx)
+    E.Conv3x3(ctx, ci, co, E.Param(ctx, wt), b, stride=stride, upsample2x=up).forward_prologue(
+        E.Tensor.from_numpy(ctx, x), aff, out)
+    assert rel(out.numpy(), want) <= gemm_bound(9 * ci)
+
+
+def test_unet_step_every_tiling(ctx, tune):
+    """A whole step: the concatenated, segmented, grouped and batched forms, LayerNorm
+    and GroupNorm partials and prologues, against the f32 products' step."""
+    net = UNet(ctx, U.random_unet())
+    inp = U.unet_input()
+    tune("gemm_split", "0")
+    want = net.forward_host(inp.x, inp.timestep)
+    for tile in TILES:
+        print(f"split unet {tile}", flush=True)
+        tune("gemm_split", tile)
+        # both are f32 results of one network, each within 2.5e-6 of its 64-bit value
+        assert rel(net.forward_host(inp.x, inp.timestep), want) <= 5e-6
