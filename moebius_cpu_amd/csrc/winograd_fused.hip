@@ -514,6 +514,25 @@ void launch_fused(Context &ctx, const FArgs &a) {
     wino_mend_kernel<<<grid, kFThreads, 0, ctx.stream>>>(a, UP, PRO);
 }
 
+// Where this kernel is faster than the three (whose plane GEMM runs at about 150
+// TFLOP/s in split products), both modelled in us. This one: rounds of one workgroup
+// per CU, 3.6 us for each 16 input channels and 6 for the output transform, 8 for
+// the two launches, and the weights' reordering where the caller has no copy. The
+// three: V and M of 16 planes at 4 TB/s, the products, 12 for the launches. A round
+// that is nearly empty costs as much as a full one, so the line is no tile count:
+// 2x64x64x512 fills one round (150 -> 125 us) and one 64x64x512 half of it (83
+// against 125); 108x148x256 97 -> 71 us; 512x512x128 takes 8 rounds and 251 us
+// against 480, 128x128x512 2 and 251 against 300. Up to the measured 512 channels.
+bool fused_is_faster(int64_t tiles, int c_in, int c_out, int cus, bool have_uf) {
+    if (c_in > 512 || c_out > 512) return false;
+    const int64_t items = ceil_div(tiles, kFT) * (c_out / kFC);
+    const double fused = 8.0 + double(ceil_div(items, int64_t(cus))) * (6.0 + 3.6 * c_in / kFK) +
+                         (have_uf ? 0.0 : 3.0 + double(winograd_fused_bytes(c_out, c_in)) / 1.8e6);
+    const double planes = 16.0 * double(tiles);
+    const double three = 12.0 + planes * 4.0 * (c_in + c_out) / 4e6 + planes * 2.0 * c_in * c_out / 150e6;
+    return fused < three;
+}
+
 }  // namespace
 
 size_t winograd_fused_bytes(int c_out, int c_in) { return size_t(16) * c_out * c_in * 6; }
@@ -533,14 +552,6 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
                             float *out, const float *residual2, GnPartials *gn) {
     if (gn) gn->rows = 0;
     if (ctx.tune.wino_fused == 0 || c_in % 32 || c_out % kFC) return false;
-    // Where it is faster (A/B per conv on MI355X, three kernels -> this one):
-    // 512x512x128 746 -> 419 us, 256x256x256 552 -> 401, the same upsampled
-    // 1824 -> 1352, 128x128x512 437 -> 402, the same upsampled 1471 -> 1335;
-    // slower on small maps, where the batched plane GEMM fills the chip at 83%
-    // of f32 MFMA peak and the V / M traffic is small: 64x64x512 100 -> 117 us,
-    // the UNet's 2x64x64x320 92 -> 124, 2x32x32x640 upsampled 281 -> 348. So:
-    // at least 4096 tiles, up to the measured 512 channels.
-    if (ctx.tune.wino_fused < 0 && (c_in > 512 || c_out > 512)) return false;
     if (!aligned16(x) || !aligned16(u) || !aligned16(out) || !aligned16(bias) || !aligned16(residual2)) return false;
     if (prologue && (!aligned16(prologue->scale) || !aligned16(prologue->shift))) return false;
     const int64_t x_bytes = int64_t(n) * h * w * c_in * 4, u_bytes = int64_t(winograd_fused_bytes(c_out, c_in));
@@ -550,7 +561,7 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
     g.h = h, g.w = w, g.hi = h << up, g.wi = w << up;
     g.th = (g.hi + 1) / 2, g.tw = (g.wi + 1) / 2;
     const int64_t tiles = int64_t(n) * g.th * g.tw;
-    if (ctx.tune.wino_fused < 0 && tiles < 4096) return false;
+    if (ctx.tune.wino_fused < 0 && !fused_is_faster(tiles, c_in, c_out, ctx.cu_count, uf != nullptr)) return false;
     if (tiles == 0) return true;
     g.tiles = int(tiles);
     const int64_t blocks = ceil_div(tiles, kFT) * (c_out / kFC);

@@ -157,3 +157,23 @@ def test_unet_step_every_tiling(ctx, tune):
         tune("gemm_split", tile)
         # both are f32 results of one network, each within 2.5e-6 of its 64-bit value
         assert rel(net.forward_host(inp.x, inp.timestep), want) <= 5e-6
+
+
+# the rule's line: one full round of workgroups, half a round, and one workgroup past a round
+@pytest.mark.parametrize("n,h,w,ci,co,fused", [(2, 64, 64, 512, 512, 1), (1, 64, 64, 512, 512, 0),
+                                               (1, 108, 148, 256, 256, 1), (1, 96, 98, 256, 512, 0)])
+def test_winograd_rule(ctx, tune, n, h, w, ci, co, fused):
+    rng = np.random.default_rng(n + ci)
+    x = E.Tensor.from_numpy(ctx, rng.standard_normal((n, h, w, ci), dtype=np.float32))
+    wt = rng.standard_normal((co, 3, 3, ci), dtype=np.float32) / np.float32(np.sqrt(9 * ci))
+    conv = E.Conv3x3(ctx, ci, co, E.Param(ctx, wt), winograd=True)
+
+    def run(v):
+        tune("wino_fused", v)
+        out = E.Tensor(ctx)
+        conv.forward(x, out)
+        return out.numpy()
+
+    print(f"wino rule {n}x{h}x{w} {ci}->{co}", flush=True)
+    got = run(-1)
+    assert np.array_equal(got, run(fused)) and rel(run(1 - fused), got) <= 2e-6
