@@ -81,6 +81,10 @@ __global__ void mfma_probe_kernel(const float *a, const float *b, float *d) {
 
 }  // namespace
 
+bool exact_reads_widened(const Context &ctx, int64_t rows, int n, int k, bool conv) {
+    return ctx.precision == Precision::Exact && !split_plan_for(ctx, rows, n, k, 1, conv).tm;
+}
+
 void conv1x1(Context &ctx, const float *x, int64_t pixels, int c_in, const void *weight, WeightType wt, int c_out,
              const float *bias, const float *residual, float *out, GemmEpilogue epi, const ResidualAffine *raff,
              const float *residual2, GnPartials *gn, const ResidualAffine *x_aff, const float *x2, int c2,

@@ -402,6 +402,14 @@ inline SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int cus, int batch,
     return best;
 }
 
+// The same under the context's tuning (gemm_split; gemm_plan forces an f32 tiling).
+inline SplitPlan split_plan_for(const Context &ctx, int64_t M, int N, int K, int batch, bool conv) {
+    ShapePlan forced;
+    if (!ctx.tune.gemm_split || K % 4 || forced_plan(ctx.tune, int(M), N, K, forced)) return SplitPlan{};
+    if (ctx.tune.split_tm) return SplitPlan{ctx.tune.split_tm, ctx.tune.split_bn, ctx.tune.split_wm, ctx.tune.split_wk};
+    return plan_split(M, N, K, ctx.cu_count, batch, conv);
+}
+
 template <int TM, int BN, int WM, int WK, int MODE, int PRO, bool F16>
 void launch_split_cfg(Context &ctx, GemmArgs &p, GemmEpilogue epi, int batch) {
     constexpr int BM = TM * WM, NT = 64 * WM * WK;
@@ -448,12 +456,9 @@ bool launch_split_tile(Context &ctx, GemmArgs &p, const SplitPlan &s, GemmEpilog
 // A vector A operand (checked by the caller) and vector weight rows.
 template <int MODE, int PRO>
 bool launch_split(Context &ctx, GemmArgs &p, WeightType wt, GemmEpilogue epi, int batch) {
-    ShapePlan forced;
-    if (!ctx.tune.gemm_split || forced_plan(ctx.tune, p.M, p.N, p.K, forced)) return false;
+    const SplitPlan s = split_plan_for(ctx, p.M, p.N, p.K, batch, MODE >= kConvAligned);
     const int esz = wt == kF16 ? 2 : 4;
-    if (p.K % 4 || p.ldb % 4 || reinterpret_cast<uintptr_t>(p.b) % (4 * esz) || (batch > 1 && p.b_bs % 4)) return false;
-    SplitPlan s = plan_split(p.M, p.N, p.K, ctx.cu_count, batch, MODE >= kConvAligned);
-    if (ctx.tune.split_tm) s = SplitPlan{ctx.tune.split_tm, ctx.tune.split_bn, ctx.tune.split_wm, ctx.tune.split_wk};
+    if (!s.tm || p.ldb % 4 || reinterpret_cast<uintptr_t>(p.b) % (4 * esz) || (batch > 1 && p.b_bs % 4)) return false;
     return wt == kF16 ? launch_split_tile<0, MODE, PRO, true>(ctx, p, s, epi, batch)
                       : launch_split_tile<0, MODE, PRO, false>(ctx, p, s, epi, batch);
 }

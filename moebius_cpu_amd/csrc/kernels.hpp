@@ -41,6 +41,11 @@ void math_eval(Context &ctx, int which, const float *x, int64_t len, float *y);
 // dst [n][item] = src [item]: one item repeated over a batch.
 void tile_items(Context &ctx, const float *src, int64_t item, int n, float *dst);
 
+// Whether EXACT arithmetic takes this GEMM (weight rows n, of k values) to the f32
+// instructions, whose kernels prefer an f16-stored weight's f32 widening; the split
+// bf16 kernels prefer the f16 values. Either copy gives the same bits.
+bool exact_reads_widened(const Context &ctx, int64_t rows, int n, int k, bool conv);
+
 // ---- normalisation (norm.hip) ----
 // add (optional): per item and channel, item b's row at add + b * add_ld (add_ld 0: c).
 // x2 (optional): the input is [x | x2] per pixel, x holding the first c - c2

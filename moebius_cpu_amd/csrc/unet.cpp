@@ -76,7 +76,7 @@ WeightStore::WeightStore(Context &ctx, const NamedTensor *t, int count, bool wid
         e.host_dtype = t[i].dtype;
         if (!m_.emplace(t[i].name, e).second) fail(kInvalidArgument, std::string("duplicate tensor ") + t[i].name);
     }
-    // f32 widenings of the f16-stored (GEMM) weights, for EXACT arithmetic
+    // f32 widenings of the f16-stored (GEMM) weights, for EXACT arithmetic on the f32 instructions
     size_t wide = 0;
     for (auto &kv : m_)
         if (widen && kv.second.d.wt == kF16) wide += (size_t(kv.second.d.numel) * 4 + 255) & ~size_t(255);
@@ -223,7 +223,7 @@ struct Lin {  // Conv1x1 (src/engine/conv.rs:28-55)
     }
     void fwd(Env &e, const float *x, int64_t px, float *out, const float *res = nullptr,
              GemmEpilogue epi = GemmEpilogue::None) const {
-        const DParam wd = w.at(e.ctx);
+        const DParam wd = w.at(e.ctx, px, co, ci);
         conv1x1(e.ctx, x, px, ci, wd.p, wd.wt, co, b, res, out, epi);
     }
     DT fwd(Env &e, const DT &x, const DT *res = nullptr, GemmEpilogue epi = GemmEpilogue::None) const {
@@ -235,7 +235,7 @@ struct Lin {  // Conv1x1 (src/engine/conv.rs:28-55)
     // LayerNorm that reads it next.
     DT fwd_lnp(Env &e, const DT &x, LnRowPartials *lnp) const {
         DT out = e.pool.tensor(x.n, x.h, x.w, co);
-        const DParam wd = w.at(e.ctx);
+        const DParam wd = w.at(e.ctx, x.px(), co, ci);
         conv1x1(e.ctx, x.p, x.px(), ci, wd.p, wd.wt, co, b, nullptr, out.p, GemmEpilogue::None, nullptr, nullptr,
                 nullptr, nullptr, nullptr, 0, lnp);
         return out;
@@ -243,7 +243,7 @@ struct Lin {  // Conv1x1 (src/engine/conv.rs:28-55)
     // The same of [xa | xb] per pixel, read from the two tensors.
     DT fwd2(Env &e, const DT &xa, const DT &xb) const {
         DT out = e.pool.tensor(xa.n, xa.h, xa.w, co);
-        const DParam wd = w.at(e.ctx);
+        const DParam wd = w.at(e.ctx, xa.px(), co, ci);
         conv1x1(e.ctx, xa.p, xa.px(), ci, wd.p, wd.wt, co, b, nullptr, out.p, GemmEpilogue::None, nullptr, nullptr,
                 nullptr, nullptr, xb.p, xb.c);
         return out;
@@ -258,7 +258,7 @@ struct Lin {  // Conv1x1 (src/engine/conv.rs:28-55)
         xa.shift = ss + int64_t(x.n) * x.c;
         xa.silu = false;
         xa.rows_per_item = x.h * x.w;
-        const DParam wd = w.at(e.ctx);
+        const DParam wd = w.at(e.ctx, x.px(), co, ci);
         conv1x1(e.ctx, x.p, x.px(), ci, wd.p, wd.wt, co, b, nullptr, out.p, GemmEpilogue::None, nullptr, nullptr,
                 nullptr, &xa, nullptr, 0, lnp);
         return out;
@@ -268,7 +268,7 @@ struct Lin {  // Conv1x1 (src/engine/conv.rs:28-55)
     DT fwd_gnp(Env &e, const DT &x, const DT *res = nullptr) const {
         DT out = e.pool.tensor(x.n, x.h, x.w, co);
         GnPartials gp = gn_request(e, x, co);
-        const DParam wd = w.at(e.ctx);
+        const DParam wd = w.at(e.ctx, x.px(), co, ci);
         conv1x1(e.ctx, x.p, x.px(), ci, wd.p, wd.wt, co, b, res ? res->p : nullptr, out.p, GemmEpilogue::None, nullptr,
                 nullptr, &gp);
         gn_attach(e, out, gp);
@@ -353,7 +353,7 @@ struct DwConv2d {
     // res2: added last (the resnet's shortcut). out: caller's buffer or a new tensor.
     DT fwd(Env &e, const DT &x, const float *res2 = nullptr, float *out_p = nullptr) const {
         DT mid = e.pool.tensor(x.n, x.h, x.w, x.c);
-        const DParam wd = pw.w.at(e.ctx);
+        const DParam wd = pw.w.at(e.ctx, x.px(), co, pw.ci);
         const bool h16 = dw_h16(e, wd) && depthwise3x3_h16(e.ctx, x.p, x.n, x.h, x.w, x.c, dw, dwb, 1, mid.p);
         if (!h16) depthwise3x3(e.ctx, x.p, x.n, x.h, x.w, x.c, dw, dwb, 1, mid.p);
         DT out = out_p ? DT{out_p, x.n, x.h, x.w, co} : e.pool.tensor(x.n, x.h, x.w, co);
@@ -382,7 +382,7 @@ struct DwConv2d {
         aff.shift = ss + int64_t(xa.n) * cc;
         aff.silu = true;
         DT mid = e.pool.tensor(xa.n, xa.h, xa.w, cc);
-        const DParam wd = pw.w.at(e.ctx);
+        const DParam wd = pw.w.at(e.ctx, xa.px(), co, pw.ci);
         const bool h16 = dw_h16(e, wd) &&
                          depthwise3x3_h16(e.ctx, xa.p, xa.n, xa.h, xa.w, cc, dw, dwb, 1, mid.p, &aff, xb.p, xb.c);
         if (!h16) depthwise3x3(e.ctx, xa.p, xa.n, xa.h, xa.w, cc, dw, dwb, 1, mid.p, &aff, xb.p, xb.c);
@@ -406,7 +406,7 @@ struct DwConv2d {
         aff.shift = ss + int64_t(x.n) * x.c;
         aff.silu = true;
         DT mid = e.pool.tensor(x.n, x.h, x.w, x.c);
-        const DParam wd = pw.w.at(e.ctx);
+        const DParam wd = pw.w.at(e.ctx, x.px(), co, pw.ci);
         const bool h16 = dw_h16(e, wd) && depthwise3x3_h16(e.ctx, x.p, x.n, x.h, x.w, x.c, dw, dwb, 1, mid.p, &aff);
         if (!h16) depthwise3x3(e.ctx, x.p, x.n, x.h, x.w, x.c, dw, dwb, 1, mid.p, &aff);
         DT out = out_p ? DT{out_p, x.n, x.h, x.w, co} : e.pool.tensor(x.n, x.h, x.w, co);
@@ -827,13 +827,13 @@ struct MixTransformer {
             e.pool.recycle(t);
         }
         DT g = e.pool.tensor(a.n, a.h, a.w, hidden);
-        const DParam pwd = point.w.at(e.ctx);
+        const DParam pwd = point.w.at(e.ctx, a.px(), point.co, point.ci);
         const bool h16 = dw_h16(e, pwd) && depthwise3x3_h16(e.ctx, a.p, a.n, a.h, a.w, a.c, dw, dwb, 2, g.p);
         if (!h16) depthwise3x3(e.ctx, a.p, a.n, a.h, a.w, a.c, dw, dwb, 2, g.p);
         e.pool.recycle(a);
         DT u;
         // u, read only by proj_out: f16 as well when proj_out's weight is
-        const DParam powd = proj_out.w.at(e.ctx);
+        const DParam powd = proj_out.w.at(e.ctx, g.px(), proj_out.co, proj_out.ci);
         const bool u16 = h16 && powd.wt == kF16;
         if (h16) {
             u = e.pool.tensor(g.n, g.h, g.w, point.co);
@@ -890,9 +890,10 @@ struct Conv3 {
             conv3x3_winograd(e.ctx, x.p, x.n, x.h, x.w, x.c, u16, kF16, c, b, up, nullptr, out.p);
         else if (u)
             conv3x3_winograd(e.ctx, x.p, x.n, x.h, x.w, x.c, u, kF32, c, b, up, nullptr, out.p);
-        else
-            conv3x3(e.ctx, x.p, x.n, x.h, x.w, x.c, w.at(e.ctx).p, w.at(e.ctx).wt, c, b, stride, pad, up, nullptr,
-                    out.p);
+        else {
+            const DParam wd = w.at(e.ctx, out.px(), c, 9 * x.c, true);
+            conv3x3(e.ctx, x.p, x.n, x.h, x.w, x.c, wd.p, wd.wt, c, b, stride, pad, up, nullptr, out.p);
+        }
         return out;
     }
 };
@@ -1044,7 +1045,7 @@ class UNetDevice {
         silu_tile(ctx_, temb.p, TIME_EMBED, b, temb_silu);
         // all resnets' time projections: tp [b][temb_total_]
         float *tp = pool_.floats(int64_t(b) * temb_total_);
-        const bool t32 = temb_w32_ && ctx_.precision == Precision::Exact;
+        const bool t32 = temb_w32_ && exact_reads_widened(ctx_, b, temb_total_, TIME_EMBED, false);
         conv1x1(ctx_, temb_silu, b, TIME_EMBED, t32 ? temb_w32_ : temb_w_, t32 ? kF32 : temb_wt_, temb_total_, temb_b_,
                 nullptr, tp);
 
