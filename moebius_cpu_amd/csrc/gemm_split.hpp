@@ -418,9 +418,7 @@ void launch_split_cfg(Context &ctx, GemmArgs &p, GemmEpilogue epi, int batch) {
     constexpr bool kSquare = Waves<BM, BN, WM, 1, WK, 16>::kFixedQuads;
     const unsigned tiles = unsigned(ceil_div(p.M, BM) * ceil_div(p.N, BN));
     log_gemm(ctx, "split", p, BM, BN, 1, MODE, PRO, F16, epi, batch, WM, 1, WK);
-    char family[64];
-    if (ctx.tune.gemm_time) std::snprintf(family, sizeof family, "f32 split %dx%dx%d", p.M, p.N, p.K);
-    const GemmTimer timer(ctx, family, p, BM, BN, WM, 1, WK, 1, MODE, batch);
+    const GemmTimer timer(ctx, "f32 split", p, BM, BN, WM, 1, WK, 1, MODE, batch);
     p.k_split = p.K;
     p.vec_out = out_vec_ok(p, BM);
     gn_partials_plan(p, BM, BN, 1, batch, kSquare);
