@@ -225,6 +225,19 @@ int32_t mh_conv3x3_winograd(MhContext *ctx, const float *x, uint32_t n, uint32_t
                             const float *prologue_scale, const float *prologue_shift, uint32_t prologue_silu,
                             float *out);
 
+/* No counterpart in the reference: mh_conv3x3_winograd with a residual added last
+ * (residual2, or NULL; not out) and the GroupNorm statistics that the one-kernel
+ * path writes, which this library's VAE hands to the next GroupNorm; exposed so they
+ * can be checked. part as in mh_conv1x1_gn_partials: per block of *rows output pixels
+ * in tile order, each channel's sum and sum of squares of the values stored (needs
+ * ceil(tiles / 32) * c_out * 2 floats, 16-byte aligned). *rows is 0 (part not written)
+ * where the conv takes the three-kernel path or its blocks would straddle items. */
+int32_t mh_conv3x3_winograd_gn_partials(MhContext *ctx, const float *x, uint32_t n, uint32_t h, uint32_t w,
+                                        uint32_t c_in, const float *u, uint32_t c_out, const float *bias,
+                                        uint32_t upsample2x, const float *prologue_scale, const float *prologue_shift,
+                                        uint32_t prologue_silu, const float *residual2, float *out, float *part,
+                                        uint32_t *rows);
+
 /* src/engine/conv.rs:145-165 `Geometry::gather`: patch rows [3,3,c] of output
  * pixels first..first+count (the implicit-GEMM conv's A operand, materialised
  * for a bit-exact check). rows [count, 9*c]. */

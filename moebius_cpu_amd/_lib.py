@@ -82,6 +82,8 @@ SIGNATURES = {
     "mh_winograd_input_transform": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _vp, _vp, _u32, _vp]),
     "mh_winograd_output_transform": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _vp, _vp]),
     "mh_conv3x3_winograd": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _vp, _u32, _vp, _u32, _vp, _vp, _u32, _vp]),
+    "mh_conv3x3_winograd_gn_partials": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _vp, _u32, _vp, _u32, _vp, _vp, _u32,
+                                               _vp, _vp, _vp, _u32p]),
     "mh_im2col_gather": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _u32p, _u32, _u64, _u64, _vp]),
     "mh_depthwise3x3": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _vp, _vp, _u32, _vp]),
     "mh_depthwise3x3_fused": (_i32, [_vp, _vp, _u32, _u32, _u32, _u32, _vp, _vp, _u32, _vp, _vp, _u32, _vp]),

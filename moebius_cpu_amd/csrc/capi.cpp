@@ -447,6 +447,37 @@ int32_t mh_conv3x3_winograd(MhContext *ctx, const float *x, uint32_t n, uint32_t
     });
 }
 
+int32_t mh_conv3x3_winograd_gn_partials(MhContext *ctx, const float *x, uint32_t n, uint32_t h, uint32_t w,
+                                        uint32_t c_in, const float *u, uint32_t c_out, const float *bias,
+                                        uint32_t upsample2x, const float *prologue_scale, const float *prologue_shift,
+                                        uint32_t prologue_silu, const float *residual2, float *out, float *part,
+                                        uint32_t *rows) {
+    return guard([&] {
+        mh::Context &cc = C(ctx);
+        need(x, "x");
+        need(u, "u");
+        need(out, "out");
+        need(part, "part");
+        need(rows, "rows");
+        *rows = 0;
+        if ((prologue_scale == nullptr) != (prologue_shift == nullptr))
+            mh::fail(mh::kInvalidArgument, "prologue needs both scale and shift");
+        const uint32_t up = upsample2x != 0 ? 1 : 0;
+        MH_REQUIRE((int64_t(h) << up) * (int64_t(w) << up) < (int64_t(1) << 31), "Winograd partials: map too large");
+        mh::Affine aff;
+        aff.scale = prologue_scale;
+        aff.shift = prologue_shift;
+        aff.silu = prologue_silu != 0;
+        mh::GnPartials gp;
+        gp.part = part;
+        gp.item_rows = int((h << up) * (w << up));
+        mh::conv3x3_winograd(cc, x, dim(n, "n"), dim(h, "h"), dim(w, "w"), dim(c_in, "c_in"), u, mh::kF32,
+                             dim(c_out, "c_out"), bias, up != 0, prologue_scale ? &aff : nullptr, out, residual2,
+                             nullptr, &gp);
+        *rows = uint32_t(gp.rows);
+    });
+}
+
 int32_t mh_im2col_gather(MhContext *ctx, const float *x, uint32_t n, uint32_t h, uint32_t w, uint32_t c,
                          uint32_t stride, const uint32_t pad[4], uint32_t upsample2x, uint64_t first, uint64_t count,
                          float *rows) {

@@ -65,7 +65,8 @@ struct FArgs {
     const char *u;  // packed (wino_u_fused_kernel)
     const float *psc, *psh, *bias, *res2;
     float *out, *gnp;
-    int *sick;  // per workgroup: whether it met a sum that is infinite or NaN
+    int *sick;       // per workgroup: whether it met a sum that is infinite or NaN
+    const float *w;  // [16][co][ci], the U that u holds split
     FGeo g;
     uint32_t x_bytes, u_bytes;
     int ci, co, psilu, nco_blocks, nwork;
@@ -85,8 +86,17 @@ constexpr int kFPlanes = 16 / (kFThreads / 64);  // planes per wave
 // apart take different banks.
 __device__ __forceinline__ int vquad(int t, int q) { return (q ^ ((t >> 2) & 3)) * 4; }
 
-template <int UP, bool PRO>
+// F32: the repair, launched after each conv and done at once where no workgroup
+// flagged its sums. A part product of an infinite value with a zero part is NaN where
+// the f32 product is infinite, and a value within half a bf16 step of the largest f32
+// rounds to an infinite part: so a workgroup that met an infinite or NaN sum does its
+// items again, products, outputs and GroupNorm partials, on v_mfma_f32_32x32x2f32 with
+// the unsplit operands (256x256x128 -> 128, every value NaN: 195 us for both, 94 for the
+// conv alone; the residual is read again, so it is not the output).
+template <int UP, bool PRO, bool F32>
 __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
+    if constexpr (F32)
+        if (!a.sick[blockIdx.x]) return;
     const FGeo &g = a.g;
     const int ci = a.ci, co = a.co, nwork = a.nwork;
     __shared__ __align__(16) float lds[kLds];
@@ -98,15 +108,15 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
     // eighth of the items, so it works through few channel blocks and their U
     // panels stay in its L2, and its workgroups take every (grid / 8)-th item
     // of that range. The grid holds one workgroup per CU, and a workgroup
-    // issues its next item's first patch and U loads before the current
-    // item's last products and output transform, which hide their latency.
+    // issues its next item's first patch and U loads once the current item's
+    // sums have left their registers, half way through its output transform.
     const int ntb = nwork / a.nco_blocks;
     const int per_xcd = (nwork + 7) / 8;
     const int slots = int(gridDim.x) / 8;
     const int item_end = min(nwork, (int(blockIdx.x) % 8 + 1) * per_xcd);
     const int first = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
     if (first >= item_end) {
-        if (tid == 0) a.sick[blockIdx.x] = 0;
+        if (!F32 && tid == 0) a.sick[blockIdx.x] = 0;
         return;
     }
     const __amdgpu_buffer_rsrc_t ur = rsrc(a.u, a.u_bytes);
@@ -227,6 +237,31 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
                 acc[p][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v.q[kSplitTerm[t][0]].v,
                                                                       uu[j][kSplitTerm[t][1]], acc[p][i][j], 0, 0, 0);
     };
+    // The same on the f32 instructions: lane l holds K 4 (l / 32) .. + 3 of each half
+    // chunk, one of them per instruction.
+    auto products_f32 = [&](const float *vs, int kc) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int p = 0; p < kFPlanes; ++p) {
+                floatx4 va[2], ub[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    va[i] = *reinterpret_cast<const floatx4 *>(vs + ((kFPlanes * wave + p) * kFT + 32 * i + row) * kFK +
+                                                               vquad(row, 2 * s + kg));
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    ub[j] = *reinterpret_cast<const floatx4 *>(
+                        a.w + (int64_t(kFPlanes * wave + p) * co + co0 + 32 * j + row) * ci + kc * kFK + 8 * s + 4 * kg);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+                            acc[p][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i][t], ub[j][t], acc[p][i][j], 0, 0, 0);
+            }
+    };
     const int nk = ci / kFK;
     float sick = 0.0f;  // NaN once any sum is infinite or NaN
     int item = first;
@@ -234,7 +269,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
     setup_consumer(item);
     bf16x8 u0[2][3], u1[2][3];
     produce(0);
-    load_u(0, 0, u0);
+    if constexpr (!F32) load_u(0, 0, u0);
     for (;;) {
         const int next = item + slots;
         const bool has_next = next < item_end;
@@ -256,21 +291,25 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         // plane's U at the start of the chunk, the next chunk's first U half way.
         for (int kc = 0; kc < nk; ++kc) {
             const float *vs = lds + (kc & 1) * kVStage;
-            load_u(1, kc, u1);
-            __builtin_amdgcn_sched_barrier(0);
-            Split3 v;
-            read_v(vs, 0, 0, v);
-            products(0, 0, v, u0);
-            __builtin_amdgcn_sched_barrier(0);
-            read_v(vs, 0, 1, v);
-            products(0, 1, v, u0);
-            __builtin_amdgcn_sched_barrier(0);
-            load_u(0, min(kc + 1, nk - 1), u0);
-            read_v(vs, 1, 0, v);
-            products(1, 0, v, u1);
-            __builtin_amdgcn_sched_barrier(0);
-            read_v(vs, 1, 1, v);
-            products(1, 1, v, u1);
+            if constexpr (F32) {
+                products_f32(vs, kc);
+            } else {
+                load_u(1, kc, u1);
+                __builtin_amdgcn_sched_barrier(0);
+                Split3 v;
+                read_v(vs, 0, 0, v);
+                products(0, 0, v, u0);
+                __builtin_amdgcn_sched_barrier(0);
+                read_v(vs, 0, 1, v);
+                products(0, 1, v, u0);
+                __builtin_amdgcn_sched_barrier(0);
+                load_u(0, min(kc + 1, nk - 1), u0);
+                read_v(vs, 1, 0, v);
+                products(1, 0, v, u1);
+                __builtin_amdgcn_sched_barrier(0);
+                read_v(vs, 1, 1, v);
+                products(1, 1, v, u1);
+            }
             if (kc + 1 < nk) transform_store(kc + 1, (kc + 1) & 1);
             if (kc + 2 < nk) produce(kc + 2);
             __syncthreads();
@@ -282,14 +321,16 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         asm volatile("" : "+v"(etid));
         const int elane = etid & 63;
         float *const mw = lds + (kFPlanes * wave * kHT + 4 * (elane >> 5)) * kMS + (elane & 31);
+        if constexpr (!F32) {
 #pragma unroll
-        for (int p = 0; p < kFPlanes; ++p)
+            for (int p = 0; p < kFPlanes; ++p)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) sick = __builtin_fmaf(acc[p][i][j][v], 0.0f, sick);
+                        for (int v = 0; v < 16; ++v) sick = __builtin_fmaf(acc[p][i][j][v], 0.0f, sick);
+        }
 
         floatx4 gs{0.f, 0.f, 0.f, 0.f}, gq = gs;  // GroupNorm sums of the values stored
 #pragma unroll
@@ -308,7 +349,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
                          // again at the end, so that nothing older stays live)
                 setup_consumer(has_next ? next : item);
                 setup_producer(has_next ? next : item);
-                load_u(0, 0, u0);
+                if constexpr (!F32) load_u(0, 0, u0);
                 produce(0);
             }
             __syncthreads();
@@ -386,85 +427,15 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         __syncthreads();  // the output transform's reads of M are done before V stage 0 is written
         item = next;
     }
-    const int bad = __syncthreads_or(sick != sick);
-    if (tid == 0) a.sick[blockIdx.x] = bad;
-}
-
-// The outputs of one work item that are infinite or NaN, again in f32 on the vector
-// unit: a part product of an infinite value with a zero part is NaN where the f32
-// product is infinite, and a value within half a bf16 step of the largest f32
-// rounds to an infinite part. A kernel of its own, launched after each conv and done
-// at once where no workgroup flagged its sums (in the conv kernel's tail the same code
-// cost it registers: 353 against 274 us at 512x512x128 -> 128).
-__device__ __forceinline__ void wino_mend(const FArgs &a, int up, bool pro, int t0, int co0) {
-    const FGeo &g = a.g;
-    const int per_item = g.th * g.tw, ci = a.ci, co = a.co;
-#pragma nounroll
-    for (int e = threadIdx.x; e < kFT * kFC * 4; e += blockDim.x) {
-        const int t = t0 + e / (kFC * 4);
-        const int o = co0 + e % kFC, kk = (e / kFC) % 4;
-        if (t >= g.tiles) continue;
-        const int b = t / per_item, rem = t - b * per_item;
-        const int ty = rem / g.tw, tx = rem - ty * g.tw;
-        const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
-        if (oy >= g.hi || ox >= g.wi) continue;
-        const int64_t oi = ((int64_t(b) * g.hi + oy) * g.wi + ox) * co + o;
-        if (__builtin_fabsf(a.out[oi]) < __builtin_inff()) continue;
-        // A^T m A: nine planes with their signs, row by row, in the transform's order
-        float y = 0.0f, line = 0.0f;
-#pragma nounroll
-        for (int n = 0; n < 9; ++n) {
-            const int r = n / 3 + (kk >> 1), c4 = n % 3 + (kk & 1);
-            float m = 0.0f;
-#pragma nounroll
-            for (int c = 0; c < ci; ++c) {
-                float v = 0.0f, col = 0.0f;
-#pragma nounroll
-                for (int q = 0; q < 4; ++q) {
-                    // V of plane (r, c4): rows pr and columns pc of the patch with their signs
-                    const int qr = q & 1, qc = q >> 1;
-                    const int pr = r == 0 ? 2 * qr : r == 1 ? 1 + qr : r == 2 ? 2 - qr : 1 + 2 * qr;
-                    const int pc = c4 == 0 ? 2 * qc : c4 == 1 ? 1 + qc : c4 == 2 ? 2 - qc : 1 + 2 * qc;
-                    const int iy = 2 * ty + pr - 1, ix = 2 * tx + pc - 1;
-                    float dv = 0.0f;
-                    if (iy >= 0 && iy < g.hi && ix >= 0 && ix < g.wi) {
-                        dv = a.x[((int64_t(b) * g.h + (iy >> up)) * g.w + (ix >> up)) * ci + c];
-                        if (pro) {
-                            dv = __builtin_fmaf(dv, a.psc[int64_t(b) * ci + c], a.psh[int64_t(b) * ci + c]);
-                            if (a.psilu) dv = ref_silu(dv);
-                        }
-                    }
-                    col = !qr ? dv : r == 1 ? col + dv : col - dv;
-                    if (qr) v = !qc ? col : c4 == 1 ? v + col : v - col;
-                }
-                const char *blk = a.u + ((int64_t(4 * r + c4) * (ci / kFK) + c / kFK) * (co / 32) + o / 32) * 3 * kUBlk +
-                                  (((o % 32) + 32 * ((c % kFK) / 8)) * 8 + c % 8) * 2;
-                float uv = float(*reinterpret_cast<const __bf16 *>(blk + 2 * kUBlk));
-                uv = float(*reinterpret_cast<const __bf16 *>(blk + kUBlk)) + uv;
-                uv = float(*reinterpret_cast<const __bf16 *>(blk)) + uv;
-                m = __builtin_fmaf(v, uv, m);
-            }
-            line = n % 3 == 0 ? m : (kk & 1) ? line - m : line + m;
-            if (n % 3 == 2) y = n == 2 ? line : (kk >> 1) ? y - line : y + line;
-        }
-        if (a.bias) y = y + a.bias[o];
-        if (a.res2) y = y + a.res2[oi];
-        a.out[oi] = y;
+    if constexpr (!F32) {
+        const int bad = __syncthreads_or(sick != sick);
+        if (tid == 0) a.sick[blockIdx.x] = bad;
     }
 }
 
-// One workgroup per workgroup of the conv, over its items.
-__global__ __launch_bounds__(kFThreads) void wino_mend_kernel(FArgs a, int up, int pro) {
-    if (!a.sick[blockIdx.x]) return;
-    const int per_xcd = (a.nwork + 7) / 8, ntb = a.nwork / a.nco_blocks;
-    const int end = min(a.nwork, (int(blockIdx.x) % 8 + 1) * per_xcd);
-    for (int it = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8; it < end; it += int(gridDim.x) / 8)
-        wino_mend(a, up, pro != 0, it % ntb * kFT, it / ntb * kFC);
-}
-
 // u [16][co][ci] -> packed [16][ci / 16][co / 32][part][lane][8]: lane l of a block
-// holds channel l % 32, K 8 (l / 32) .. + 7. An infinite or NaN value keeps itself
-// in the first part alone, and one that rounds to infinity is cut off instead.
+// holds channel l % 32, K 8 (l / 32) .. + 7. An infinite value, or one that rounds to
+// infinity, makes the sums of its channel infinite or NaN, and the repair reads u.
 __global__ void wino_u_fused_kernel(const float *__restrict__ u, int co, int ci, char *__restrict__ uf) {
     const SplitSel sel = split_sel();
     const int64_t blocks = int64_t(16) * (ci / kFK) * (co / 32);
@@ -478,25 +449,7 @@ __global__ void wino_u_fused_kernel(const float *__restrict__ u, int co, int ci,
         const float *src = u + (int64_t(plane) * co + cb * 32 + (lane & 31)) * ci + kc * kFK + 8 * (lane >> 5);
         Split3 s;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const float a = src[2 * p], b = src[2 * p + 1];
-            split_pair(a, b, p, sel, s);
-            const float v[2] = {a, b};
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if (__builtin_fabsf(static_cast<float>(s.q[0].p[p][h])) < __builtin_inff()) continue;
-                if (__builtin_fabsf(v[h]) < __builtin_inff()) {
-                    const uint32_t bits = __builtin_bit_cast(uint32_t, v[h]);
-                    const float hi = __builtin_bit_cast(float, bits & 0xffff0000u), rest = v[h] - hi;
-                    s.q[0].p[p][h] = static_cast<__bf16>(hi);
-                    s.q[1].p[p][h] = static_cast<__bf16>(rest);
-                    s.q[2].p[p][h] = static_cast<__bf16>(rest - static_cast<float>(s.q[1].p[p][h]));
-                } else {
-                    s.q[0].p[p][h] = static_cast<__bf16>(v[h]);
-                    s.q[1].p[p][h] = s.q[2].p[p][h] = static_cast<__bf16>(0.0f);
-                }
-            }
-        }
+        for (int p = 0; p < 4; ++p) split_pair(src[2 * p], src[2 * p + 1], p, sel, s);
         char *dst = uf + blk * 3 * kUBlk + lane * 16;
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8 *>(dst + q * kUBlk) = s.q[q].v;
@@ -509,9 +462,9 @@ void launch_fused(Context &ctx, const FArgs &a) {
     // order in the kernel), no more than the items of one XCD's share need
     const int64_t per_xcd = ceil_div(a.nwork, 8);
     const unsigned grid = unsigned(8 * std::max<int64_t>(1, std::min<int64_t>(ctx.cu_count / 8, per_xcd)));
-    wino_fused_kernel<UP, PRO><<<grid, kFThreads, 0, ctx.stream>>>(a);
+    wino_fused_kernel<UP, PRO, false><<<grid, kFThreads, 0, ctx.stream>>>(a);
     MH_LAUNCH_CHECK();
-    wino_mend_kernel<<<grid, kFThreads, 0, ctx.stream>>>(a, UP, PRO);
+    wino_fused_kernel<UP, PRO, true><<<grid, kFThreads, 0, ctx.stream>>>(a);
 }
 
 // Where this kernel is faster than the three (whose plane GEMM runs at about 150
@@ -587,7 +540,7 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
                   prologue ? prologue->shift : nullptr,
                   bias, residual2,
                   out,  gnp,
-                  ctx.wino_flags,
+                  ctx.wino_flags, u,
                   g,    xb,
                   ub,   c_in,
                   c_out, prologue && prologue->silu ? 1 : 0,
