@@ -52,12 +52,13 @@ constexpr int kMS = kFC + 4;             // M row stride in LDS (floats)
 constexpr int kRed = 16 * kHT * kMS;     // GroupNorm reduction scratch, past the M exchange
 constexpr int kLds = kRed + 2 * 8 * 64;  // floats, 140 KB
 static_assert(2 * kVStage <= kLds && kRed >= kVStage, "the V stages fit, the scratch in stage 1 or past it");
-constexpr int kOob = int(0x80000000u);   // past any buffer: reads zero
+constexpr uint32_t kXEnd = 0x80000000u;  // the input buffer's extent
+constexpr int kOob = int(kXEnd);         // past any buffer: reads zero
 constexpr int kUBlk = 1024;              // bytes of one packed U block: 32 channels x 16 K of one part
 
 struct FGeo {
     int h, w, hi, wi, th, tw;
-    int tiles;  // the input's 1 GiB holds fewer than 2^23 pixels
+    int tiles;  // the input's 2 GiB hold no more than 2^24 pixels
 };
 
 struct FArgs {
@@ -68,7 +69,7 @@ struct FArgs {
     int *sick;       // per workgroup: whether it met a sum that is infinite or NaN
     const float *w;  // [16][co][ci], the U that u holds split
     FGeo g;
-    uint32_t x_bytes, u_bytes;
+    uint32_t u_bytes;
     int ci, co, psilu, nco_blocks, nwork;
 };
 
@@ -138,7 +139,12 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
     bool rowin[4], colin[4];        // pixel early, so that a patch row or column's step is never negative
     const int prow = g.w * ci * 4, pcol = ci * 4;  // bytes per source row, per pixel
     constexpr int kStep[4] = {0, 1, 2 - UP, 3 - UP};  // patch row / column k -> source offset + 1
-    const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char *>(a.x) - prow - pcol, a.x_bytes + prow + pcol);
+    // A load's checked offset is porg or kOob; the patch's step and the chunk are in its
+    // scalar offset. With the extent at kXEnd whatever the map, kOob is out of range
+    // whether the check leaves the scalar offset out, adds it or takes it off the extent
+    // (which on a map of a row or two it exceeds), and the loads that are made are inside
+    // the input by rowin and colin alone.
+    const __amdgpu_buffer_rsrc_t xr = rsrc(reinterpret_cast<const char *>(a.x) - prow - pcol, kXEnd);
     auto setup_producer = [&](int it) {
         int ptid = tid;
         asm volatile("" : "+v"(ptid));
@@ -147,7 +153,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         const int ty = rem / g.tw, tx = rem - ty * g.tw;
         vb = min(b, n_items - 1);  // a tile past the end reads nothing, but keeps its prologue loads in range
         const int sy = (2 * ty) >> UP, sx = (2 * tx) >> UP;
-        porg = ((b * g.h + sy) * g.w + sx) * pcol + 8 * (ptid & (kFK / 2 - 1));
+        porg = int(uint32_t((b * g.h + sy) * g.w + sx) * uint32_t(pcol)) + 8 * (ptid & (kFK / 2 - 1));
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int iy = 2 * ty + k - 1, ix = 2 * tx + k - 1;
@@ -520,7 +526,7 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
     const int64_t blocks = ceil_div(tiles, kFT) * (c_out / kFC);
     if (blocks >= (int64_t(1) << 30)) return false;
     const int nwork = int(blocks);
-    const uint32_t xb = uint32_t(x_bytes), ub = uint32_t(u_bytes);
+    const uint32_t ub = uint32_t(u_bytes);
     if (!uf) {  // no precomputed fused-order copy: make one in the workspace
         void *tmp = ctx.ws.get(size_t(u_bytes), ctx.stream);
         winograd_fused_weights(ctx, u, c_out, c_in, tmp);
@@ -541,9 +547,8 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
                   bias, residual2,
                   out,  gnp,
                   ctx.wino_flags, u,
-                  g,    xb,
-                  ub,   c_in,
-                  c_out, prologue && prologue->silu ? 1 : 0,
+                  g,    ub,
+                  c_in, c_out, prologue && prologue->silu ? 1 : 0,
                   c_out / kFC, nwork};
     if (up) prologue ? launch_fused<1, true>(ctx, a) : launch_fused<1, false>(ctx, a);
     else prologue ? launch_fused<0, true>(ctx, a) : launch_fused<0, false>(ctx, a);
