@@ -213,7 +213,8 @@ void winograd_fused_weights(Context &ctx, const float *u, int c_out, int c_in, v
 bool conv3x3_small_co(Context &ctx, const float *x, int n, int h, int w, int c_in, const void *weight, WeightType wt,
                       int c_out, const float *bias, const Affine *prologue, float *out, const float *residual2);
 // The whole conv in one kernel (winograd_fused.hip) for f32 u, c_in % 32 == 0,
-// c_out % 64 == 0, the input under 1 GiB and u's copy under 2 GiB; false (nothing launched) otherwise.
+// c_out % 64 == 0, the input (a row and a pixel more) and u's copy within 2 GiB; false (nothing
+// launched) otherwise. residual2 is not out.
 // uf: u in the fused order, or NULL (then made in the workspace for this call).
 // gn (optional): GroupNorm partials of out, blocks of 256 pixels (gn->rows set,
 // 0 where not written: odd output sizes, tiles per item not a multiple of 64).

@@ -513,8 +513,9 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
     if (ctx.tune.wino_fused == 0 || c_in % 32 || c_out % kFC) return false;
     if (!aligned16(x) || !aligned16(u) || !aligned16(out) || !aligned16(bias) || !aligned16(residual2)) return false;
     if (prologue && (!aligned16(prologue->scale) || !aligned16(prologue->shift))) return false;
-    const int64_t x_bytes = int64_t(n) * h * w * c_in * 4, u_bytes = int64_t(winograd_fused_bytes(c_out, c_in));
-    if (x_bytes >= (int64_t(1) << 30) || u_bytes >= (int64_t(1) << 31)) return false;
+    // the kernel's buffer starts a row and a pixel before the input
+    const int64_t x_span = (int64_t(n) * h * w + w + 1) * c_in * 4, u_bytes = int64_t(winograd_fused_bytes(c_out, c_in));
+    if (x_span > int64_t(kXEnd) || u_bytes >= (int64_t(1) << 31)) return false;
     FGeo g;
     const int up = upsample2x ? 1 : 0;
     g.h = h, g.w = w, g.hi = h << up, g.wi = w << up;
