@@ -216,8 +216,8 @@ bool conv3x3_small_co(Context &ctx, const float *x, int n, int h, int w, int c_i
 // c_out % 64 == 0, the input (a row and a pixel more) and u's copy within 2 GiB; false (nothing
 // launched) otherwise. residual2 is not out.
 // uf: u in the fused order, or NULL (then made in the workspace for this call).
-// gn (optional): GroupNorm partials of out, blocks of 256 pixels (gn->rows set,
-// 0 where not written: odd output sizes, tiles per item not a multiple of 64).
+// gn (optional): GroupNorm partials of out, blocks of 256 or 128 pixels (gn->rows set,
+// 0 where not written: odd output sizes, tiles per item not a multiple of 32).
 bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, int c_in, const float *u,
                             const void *uf, int c_out, const float *bias, bool upsample2x, const Affine *prologue,
                             float *out, const float *residual2, GnPartials *gn = nullptr);

@@ -71,6 +71,7 @@ struct FArgs {
     FGeo g;
     uint32_t u_bytes;
     int ci, co, psilu, nco_blocks, nwork;
+    int gn_halves;  // partials of 32 tiles each, not of a whole block: items of an odd number of 32 tiles
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, uint32_t bytes) {
@@ -339,6 +340,37 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         }
 
         floatx4 gs{0.f, 0.f, 0.f, 0.f}, gq = gs;  // GroupNorm sums of the values stored
+        // GroupNorm partials of this block or of each half (per channel: sum and sum of
+        // squares over its 256 or 128 pixels), for the next GroupNorm's fold in place of
+        // a statistics pass: the four threads of a wave that hold channel quad q (tiles
+        // 4w .. 4w + 3 of each half) by xor butterfly, then the eight waves in order
+        // through LDS past the M exchange.
+        auto write_partials = [&](int block) {
+#pragma unroll
+            for (int off = 16; off < 64; off <<= 1)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    gs[e] += __shfl_xor(gs[e], off, 64);
+                    gq[e] += __shfl_xor(gq[e], off, 64);
+                }
+            floatx4 *red = reinterpret_cast<floatx4 *>(lds + kRed);
+            if (elane < kFC / 4) {
+                red[wave * (kFC / 4) + elane] = gs;
+                red[(kFThreads / 64 + wave) * (kFC / 4) + elane] = gq;
+            }
+            __syncthreads();
+            if (etid < kFC / 4) {
+                floatx4 ts = red[etid], tq = red[(kFThreads / 64) * (kFC / 4) + etid];
+#pragma unroll
+                for (int w8 = 1; w8 < kFThreads / 64; ++w8) {
+                    ts = add4(ts, red[w8 * (kFC / 4) + etid]);
+                    tq = add4(tq, red[(kFThreads / 64 + w8) * (kFC / 4) + etid]);
+                }
+                float *dst = a.gnp + (int64_t(block) * co + eco0 + 4 * etid) * 2;
+                *reinterpret_cast<floatx4 *>(dst) = floatx4{ts[0], tq[0], ts[1], tq[1]};
+                *reinterpret_cast<floatx4 *>(dst + 4) = floatx4{ts[2], tq[2], ts[3], tq[3]};
+            }
+        };
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             // M [16][tile][channel] of 32 tiles through LDS: register v of lane l holds
@@ -361,74 +393,49 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
             __syncthreads();
             const int tl = etid >> 4, q = etid & 15;
             const int t = et0 + kHT * half + tl;
-            if (t >= g.tiles) continue;
-            const int b = t / per_item, rem = t - b * per_item;
-            const int ty = rem / g.tw, tx = rem - ty * g.tw;
-            const float *src = lds + tl * kMS + 4 * q;
-            floatx4 m0[4], m1[4];
+            if (t < g.tiles) {
+                const int b = t / per_item, rem = t - b * per_item;
+                const int ty = rem / g.tw, tx = rem - ty * g.tw;
+                const float *src = lds + tl * kMS + 4 * q;
+                floatx4 m0[4], m1[4];
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const floatx4 aa = *reinterpret_cast<const floatx4 *>(src + (rr * 4) * kHT * kMS);
-                const floatx4 bb = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 1) * kHT * kMS);
-                const floatx4 cc = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 2) * kHT * kMS);
-                const floatx4 dd = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 3) * kHT * kMS);
-                m0[rr] = add4(add4(aa, bb), cc);
-                m1[rr] = sub4(sub4(bb, cc), dd);
-                asm volatile("" ::: "memory");  // sixteen rows at once would not fit the registers
-            }
-            const int c = eco0 + 4 * q;
-            const floatx4 bv = a.bias ? *reinterpret_cast<const floatx4 *>(a.bias + c) : floatx4{0.f, 0.f, 0.f, 0.f};
-            floatx4 y[4];
-            y[0] = add4(add4(add4(m0[0], m0[1]), m0[2]), bv);
-            y[1] = add4(add4(add4(m1[0], m1[1]), m1[2]), bv);
-            y[2] = add4(sub4(sub4(m0[1], m0[2]), m0[3]), bv);
-            y[3] = add4(sub4(sub4(m1[1], m1[2]), m1[3]), bv);
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
-                if (oy >= g.hi || ox >= g.wi) continue;
-                const int64_t o = int64_t((b * g.hi + oy) * g.wi + ox) * co + c;
-                floatx4 rv = y[kk];
-                if (a.res2) rv = add4(rv, *reinterpret_cast<const floatx4 *>(a.res2 + o));
-                *reinterpret_cast<floatx4 *>(a.out + o) = rv;
-                if (a.gnp) {
-                    gs = add4(gs, rv);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) gq[e] = __builtin_fmaf(rv[e], rv[e], gq[e]);
+                for (int rr = 0; rr < 4; ++rr) {
+                    const floatx4 aa = *reinterpret_cast<const floatx4 *>(src + (rr * 4) * kHT * kMS);
+                    const floatx4 bb = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 1) * kHT * kMS);
+                    const floatx4 cc = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 2) * kHT * kMS);
+                    const floatx4 dd = *reinterpret_cast<const floatx4 *>(src + (rr * 4 + 3) * kHT * kMS);
+                    m0[rr] = add4(add4(aa, bb), cc);
+                    m1[rr] = sub4(sub4(bb, cc), dd);
+                    asm volatile("" ::: "memory");  // sixteen rows at once would not fit the registers
                 }
+                const int c = eco0 + 4 * q;
+                const floatx4 bv = a.bias ? *reinterpret_cast<const floatx4 *>(a.bias + c) : floatx4{0.f, 0.f, 0.f, 0.f};
+                floatx4 y[4];
+                y[0] = add4(add4(add4(m0[0], m0[1]), m0[2]), bv);
+                y[1] = add4(add4(add4(m1[0], m1[1]), m1[2]), bv);
+                y[2] = add4(sub4(sub4(m0[1], m0[2]), m0[3]), bv);
+                y[3] = add4(sub4(sub4(m1[1], m1[2]), m1[3]), bv);
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
+                    if (oy >= g.hi || ox >= g.wi) continue;
+                    const int64_t o = int64_t((b * g.hi + oy) * g.wi + ox) * co + c;
+                    floatx4 rv = y[kk];
+                    if (a.res2) rv = add4(rv, *reinterpret_cast<const floatx4 *>(a.res2 + o));
+                    *reinterpret_cast<floatx4 *>(a.out + o) = rv;
+                    if (a.gnp) {
+                        gs = add4(gs, rv);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) gq[e] = __builtin_fmaf(rv[e], rv[e], gq[e]);
+                    }
+                }
+            }
+            if (a.gnp && a.gn_halves && et0 + kHT * half < g.tiles) {
+                write_partials(et0 / kHT + half);
+                gs = gq = floatx4{0.f, 0.f, 0.f, 0.f};
             }
         }
-        if (a.gnp) {
-            // GroupNorm partials of this block (per channel: sum and sum of
-            // squares over its 256 pixels), for the next GroupNorm's fold in
-            // place of a statistics pass: the four threads of a wave that hold
-            // channel quad q (tiles 4w .. 4w + 3 of each half) by xor butterfly,
-            // then the eight waves in order through LDS past the M exchange.
-#pragma unroll
-            for (int off = 16; off < 64; off <<= 1)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    gs[e] += __shfl_xor(gs[e], off, 64);
-                    gq[e] += __shfl_xor(gq[e], off, 64);
-                }
-            floatx4 *red = reinterpret_cast<floatx4 *>(lds + kRed);
-            if (elane < kFC / 4) {
-                red[wave * (kFC / 4) + elane] = gs;
-                red[(kFThreads / 64 + wave) * (kFC / 4) + elane] = gq;
-            }
-            __syncthreads();
-            if (etid < kFC / 4) {
-                floatx4 ts = red[etid], tq = red[(kFThreads / 64) * (kFC / 4) + etid];
-#pragma unroll
-                for (int w8 = 1; w8 < kFThreads / 64; ++w8) {
-                    ts = add4(ts, red[w8 * (kFC / 4) + etid]);
-                    tq = add4(tq, red[(kFThreads / 64 + w8) * (kFC / 4) + etid]);
-                }
-                float *dst = a.gnp + (int64_t(et0 / kFT) * co + eco0 + 4 * etid) * 2;
-                *reinterpret_cast<floatx4 *>(dst) = floatx4{ts[0], tq[0], ts[1], tq[1]};
-                *reinterpret_cast<floatx4 *>(dst + 4) = floatx4{ts[2], tq[2], ts[3], tq[3]};
-            }
-        }
+        if (a.gnp && !a.gn_halves) write_partials(et0 / kFT);
         if (!has_next) break;
         __syncthreads();  // the output transform's reads of M are done before V stage 0 is written
         item = next;
@@ -535,12 +542,13 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
     } else if (!aligned16(uf)) {
         return false;
     }
-    // GroupNorm partials: blocks of 64 whole tiles (256 pixels) within one item
+    // GroupNorm partials: blocks of 64 or 32 whole tiles (256 or 128 pixels) within one item
     float *gnp = nullptr;
+    const bool halves = int64_t(g.th) * g.tw % kFT != 0;
     if (gn && gn->part && aligned16(gn->part) && g.hi % 2 == 0 && g.wi % 2 == 0 &&
-        int64_t(g.th) * g.tw % kFT == 0 && gn->item_rows == g.hi * g.wi) {
+        int64_t(g.th) * g.tw % kHT == 0 && gn->item_rows == g.hi * g.wi) {
         gnp = gn->part;
-        gn->rows = 4 * kFT;
+        gn->rows = 4 * (halves ? kHT : kFT);
     }
     const FArgs a{x,    static_cast<const char *>(uf),
                   prologue ? prologue->scale : nullptr,
@@ -550,7 +558,7 @@ bool conv3x3_winograd_fused(Context &ctx, const float *x, int n, int h, int w, i
                   ctx.wino_flags, u,
                   g,    ub,
                   c_in, c_out, prologue && prologue->silu ? 1 : 0,
-                  c_out / kFC, nwork};
+                  c_out / kFC, nwork, halves ? 1 : 0};
     if (up) prologue ? launch_fused<1, true>(ctx, a) : launch_fused<1, false>(ctx, a);
     else prologue ? launch_fused<0, true>(ctx, a) : launch_fused<0, false>(ctx, a);
     MH_LAUNCH_CHECK();

@@ -67,6 +67,8 @@ def want(x, wt, b, up, aff, res):
 
 CASES = [(1, 16, 16, 32, 64, False, False, False), (2, 16, 32, 64, 64, False, True, True),
          (1, 16, 16, 64, 128, True, False, True), (2, 13, 11, 64, 64, False, True, True),
+         # blocks that straddle items (32 and 96 tiles each): partials of 32 tiles
+         (3, 8, 16, 32, 64, False, False, True), (2, 16, 24, 64, 128, False, True, False),
          # several items per workgroup, of which one is flagged
          (1, 192, 192, 32, 64, False, False, True)]
 
@@ -82,6 +84,7 @@ def test_a_huge_finite_value(ctx, n, h, w, ci, co, up, pro, res):
     got, part, rows = conv(ctx, x, wt, b, up, aff, r)
     assert np.isfinite(got).all() and rel_l2(got, want(x, wt, b, up, aff, r)) <= 1e-5
     if (h % 2, w % 2) == (0, 0):
+        assert rows == (256 if got[0].shape[0] * got[0].shape[1] % 256 == 0 else 128)
         blocks = got[0].shape[0] * got[0].shape[1] // rows
         p = part.reshape(-1, co, 2)[:n * blocks].astype(np.float64).reshape(n, blocks, co, 2).sum(axis=1)
         g = got.astype(np.float64).reshape(n, -1, co)
