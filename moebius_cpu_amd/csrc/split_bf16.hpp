@@ -8,9 +8,16 @@
 // 5.5e-7 against 6.4e-7, K = 4608 1.07e-6 against 1.21e-6. The bf16 instructions
 // issue at 1880 TFLOP/s, so six of them at 313 TFLOP/s against 144 in f32. With the
 // five small products in a sum of their own the error is a third of the f32 chain's
-// (K = 320 0.8e-7, K = 1280 about 2e-7). The instructions read subnormal bf16 parts as
-// zero: a value's error is 2^-24 of it or 2^-126, so operands keep 24 bits down to
-// 2^-110 (1e-33).
+// (K = 320 0.8e-7, K = 1280 about 2e-7).
+//
+// bf16 ends at 2^-133 (its subnormals count), so an operand keeps its 24 bits down to
+// 2^-110 and an error of 2^-134 below. That is more than f32 rounding only in sums that
+// are small themselves: of a sum s of K products the share is at most 2^-134 times the
+// absolute sums of its two operands' K values over s, under 2^-26 while s is at least
+// 2^-72 and those sums below 2^36. So the kernels take a sum that is smaller and not
+// zero, as one that is infinite or NaN, for one to be redone on the f32 instructions
+// (SplitProbe). Scaling every operand by 2^16 before it is split keeps all bits without
+// that, and cost 1 to 3% (UNet step with CFG 6.21 -> 6.40 ms).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -60,6 +67,21 @@ __device__ __forceinline__ void split_pair(float a, float b, int e, const SplitS
     b = __builtin_amdgcn_fdot2_f32_bf16(s.q[1].p[e], sel.e1, b, false);
     s.q[2].p[e] = round_pair(a, b);
 }
+
+// Whether any of the sums seen is infinite, NaN, or too small for its operands' bits.
+struct SplitProbe {
+    float sick = 0.0f;             // NaN once a sum is infinite or NaN
+    uint32_t least = 0xffffffffu;  // the smallest 2 * |bits| - 1: a zero counts as the largest
+    __device__ __forceinline__ void see(float s) {
+        sick = __builtin_fmaf(s, 0.0f, sick);
+        const uint32_t b = (__builtin_bit_cast(uint32_t, s) << 1) - 1;
+        least = b < least ? b : least;
+    }
+    __device__ __forceinline__ bool bad() const {
+        constexpr uint32_t kLeast = (127u - 72u) << 24;  // 2^-72
+        return sick != sick || least < kLeast - 1;
+    }
+};
 
 // Part of a product term t = 0..5 in the order they are summed: {part of A, part of B}.
 constexpr int kSplitTerm[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};

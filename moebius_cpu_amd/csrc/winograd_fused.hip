@@ -66,7 +66,7 @@ struct FArgs {
     const char *u;  // packed (wino_u_fused_kernel)
     const float *psc, *psh, *bias, *res2;
     float *out, *gnp;
-    int *sick;       // per workgroup: whether it met a sum that is infinite or NaN
+    int *sick;       // per workgroup: whether it met a sum to be redone (SplitProbe)
     const float *w;  // [16][co][ci], the U that u holds split
     FGeo g;
     uint32_t u_bytes;
@@ -91,10 +91,11 @@ __device__ __forceinline__ int vquad(int t, int q) { return (q ^ ((t >> 2) & 3))
 // F32: the repair, launched after each conv and done at once where no workgroup
 // flagged its sums. A part product of an infinite value with a zero part is NaN where
 // the f32 product is infinite, and a value within half a bf16 step of the largest f32
-// rounds to an infinite part: so a workgroup that met an infinite or NaN sum does its
-// items again, products, outputs and GroupNorm partials, on v_mfma_f32_32x32x2f32 with
-// the unsplit operands (256x256x128 -> 128, every value NaN: 195 us for both, 94 for the
-// conv alone; the residual is read again, so it is not the output).
+// rounds to an infinite part; and the sums of operands below 2^-110 lack bits
+// (split_bf16.hpp). So a workgroup that met such a sum does its items again, products,
+// outputs and GroupNorm partials, on v_mfma_f32_32x32x2f32 with the unsplit operands
+// (256x256x128 -> 128, every value NaN: 195 us for both, 94 for the conv alone; the
+// residual is read again, so it is not the output).
 template <int UP, bool PRO, bool F32>
 __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
     if constexpr (F32)
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
             }
     };
     const int nk = ci / kFK;
-    float sick = 0.0f;  // NaN once any sum is infinite or NaN
+    bool sick = false;
     int item = first;
     setup_producer(item);
     setup_consumer(item);
@@ -328,17 +329,6 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         asm volatile("" : "+v"(etid));
         const int elane = etid & 63;
         float *const mw = lds + (kFPlanes * wave * kHT + 4 * (elane >> 5)) * kMS + (elane & 31);
-        if constexpr (!F32) {
-#pragma unroll
-            for (int p = 0; p < kFPlanes; ++p)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) sick = __builtin_fmaf(acc[p][i][j][v], 0.0f, sick);
-        }
-
         floatx4 gs{0.f, 0.f, 0.f, 0.f}, gq = gs;  // GroupNorm sums of the values stored
         // GroupNorm partials of this block or of each half (per channel: sum and sum of
         // squares over its 256 or 128 pixels), for the next GroupNorm's fold in place of
@@ -411,10 +401,20 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
                 const int c = eco0 + 4 * q;
                 const floatx4 bv = a.bias ? *reinterpret_cast<const floatx4 *>(a.bias + c) : floatx4{0.f, 0.f, 0.f, 0.f};
                 floatx4 y[4];
-                y[0] = add4(add4(add4(m0[0], m0[1]), m0[2]), bv);
-                y[1] = add4(add4(add4(m1[0], m1[1]), m1[2]), bv);
-                y[2] = add4(sub4(sub4(m0[1], m0[2]), m0[3]), bv);
-                y[3] = add4(sub4(sub4(m1[1], m1[2]), m1[3]), bv);
+                y[0] = add4(add4(m0[0], m0[1]), m0[2]);
+                y[1] = add4(add4(m1[0], m1[1]), m1[2]);
+                y[2] = sub4(sub4(m0[1], m0[2]), m0[3]);
+                y[3] = sub4(sub4(m1[1], m1[2]), m1[3]);
+                SplitProbe probe;  // every plane is in one of the four
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    if constexpr (!F32) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) probe.see(y[kk][e]);
+                    }
+                    y[kk] = add4(y[kk], bv);
+                }
+                sick = sick || probe.bad();
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) {
                     const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
         item = next;
     }
     if constexpr (!F32) {
-        const int bad = __syncthreads_or(sick != sick);
+        const int bad = __syncthreads_or(sick);
         if (tid == 0) a.sick[blockIdx.x] = bad;
     }
 }

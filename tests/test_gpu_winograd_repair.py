@@ -1,7 +1,8 @@
 """The one-kernel Winograd conv (csrc/winograd_fused.hip) where split sums are not
-finite: the workgroups that met one do their items again on the f32 instructions, so
-outputs and GroupNorm partials are what the f32 products give, for odd values in the
-input and in the weights, with the residual, the prologue and the upsample."""
+finite, or too small for their operands' bits: the workgroups that met one do their
+items again on the f32 instructions, so outputs and GroupNorm partials are what the
+f32 products give, for odd values in the input and in the weights, with the residual,
+the prologue and the upsample."""
 from __future__ import annotations
 
 import ctypes
@@ -137,3 +138,25 @@ def test_the_repair_is_bounded(ctx, value):
     base, odd = us(x), us(np.full_like(x, value))
     print(f"repair: {base:.0f} us finite, {odd:.0f} us all {value}", flush=True)
     assert odd <= 6 * base + 200  # the split conv and the f32 one, and the host's jitter
+
+
+# bf16 holds 24 bits of an operand down to 2^-110; an f32 sum's last bit is at 2^-149 at the least
+@pytest.mark.parametrize("exponent", [-105, -114, -119])
+@pytest.mark.parametrize("where", ["input", "half", "weights"])
+def test_small_operands(ctx, exponent, where):
+    """The whole input, its right half beside values around 1, or the weights."""
+    h, w, ci, co = 16, 48, 64, 64
+    x, wt, _, _, _ = inputs(1, h, w, ci, co, False, False, False)
+    scale = np.float32(2.0 ** exponent)
+    if where == "weights":
+        wt *= scale
+    else:
+        x[:, :, w // 2 if where == "half" else 0:] *= scale
+    got = conv(ctx, x, wt, None)[0].astype(np.float64) * 2.0 ** -exponent
+    xp = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    ref = sum(xp[:, ky:ky + h, kx:kx + w] @ wt[:, ky, kx].T.astype(np.float64)
+              for ky in range(3) for kx in range(3)) * 2.0 ** -exponent
+    if where == "half":  # the tiles that touch no value around 1
+        got, ref = got[:, :, w // 2 + 2:], ref[:, :, w // 2 + 2:]
+    # as for ordinary values: a sum of 2^-119 and more rounds to 2^-30 of it or its 24 bits
+    assert rel_l2(got, ref) <= 8 * 2.0 ** -24
