@@ -698,9 +698,7 @@ struct Waves {
     }
 };
 
-struct NoMend {
-    __device__ void operator()(float *) const {}
-};
+struct NoRedo {};
 
 // Four columns of the C tile's WK partial sums (SLAB floats apart), in group order.
 template <int WK, int SLAB>
@@ -720,13 +718,13 @@ __device__ __forceinline__ float4 sum_groups(const float *c) {
 // of wave (wm, wn, wk) holds row acc_row(v, l), column l % MF of its group's
 // partial sum; the K groups' tiles are added in LDS, then each thread finishes
 // four adjacent columns of a row at a time (16-byte loads and stores), or one
-// element at a time where that is not possible. mend (optional): called with the
-// whole C tile where any thread passes bad, before it is finished.
+// element at a time where that is not possible. redo (optional): called by every wave,
+// for its block's sums once more, where any thread passes bad.
 template <int BM, int BN, int WM, int WN, int WK, int MF, int EPI, bool SPLIT, bool FSILU = false,
-          bool OUT16 = false, typename Acc, int FM, int FN, typename Mend = NoMend>
+          bool OUT16 = false, typename Acc, int FM, int FN, typename Redo = NoRedo>
 __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const Acc (&acc)[FM][FN], int m0, int n0,
                                            int z, const float *ln_st = nullptr, bool bad = false,
-                                           const Mend &mend = Mend()) {
+                                           const Redo &redo = Redo()) {
     using MI = Mf<MF>;
     using L = Waves<BM, BN, WM, WN, WK, MF>;
     constexpr int NT = L::kThreads;
@@ -738,7 +736,7 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wm, wn, wk;
     L::index(wave, wm, wn, wk);
-    {
+    auto put = [&](const Acc (&sums)[FM][FN]) {
         float *slab = smem + wk * (BM * CS);
         const int r0 = wm * L::TM, c0 = wn * L::TN + (lane % MF);
 #pragma unroll
@@ -747,14 +745,20 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const
             for (int j = 0; j < FN; ++j)
 #pragma unroll
                 for (int v = 0; v < MI::kAccRegs; ++v)
-                    slab[(r0 + i * MF + MI::acc_row(v, lane)) * CS + c0 + j * MF] = acc[i][j][v];
+                    slab[(r0 + i * MF + MI::acc_row(v, lane)) * CS + c0 + j * MF] = sums[i][j][v];
+    };
+    put(acc);
+    if constexpr (std::is_same_v<Redo, NoRedo>) {
+        __syncthreads();
+    } else if (__builtin_expect(__syncthreads_or(bad), 0)) {
+        Acc sums[FM][FN];
+        redo(sums);
+        put(sums);
+        __syncthreads();
     }
-    int any_bad = 0;
-    if constexpr (std::is_same_v<Mend, NoMend>) __syncthreads();
-    else any_bad = __syncthreads_or(bad);
     // K groups' partial tiles: summed in group order as the store pass reads them, or
     // here into the first where the tile is needed whole.
-    const bool summed = WK == 1 || p.vec_out != 1 || any_bad;
+    const bool summed = WK == 1 || p.vec_out != 1;
     if constexpr (WK > 1) {
         if (summed) {
             constexpr int C4 = BN / 4;
@@ -762,12 +766,6 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, float *smem, const
                 const int rr = e / C4, cc = (e - rr * C4) * 4;
                 *reinterpret_cast<float4 *>(smem + rr * CS + cc) = sum_groups<WK, BM * CS>(smem + rr * CS + cc);
             }
-            __syncthreads();
-        }
-    }
-    if constexpr (!std::is_same_v<Mend, NoMend>) {
-        if (any_bad) {
-            mend(smem);
             __syncthreads();
         }
     }

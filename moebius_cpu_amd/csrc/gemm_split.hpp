@@ -27,39 +27,55 @@ namespace {
 
 constexpr int kSK = 32;  // K per matrix instruction, and per wave group and LDS stage
 
-// One output element in f32 on the vector unit, k_begin..k_end in order: for
-// elements whose split sum is not finite. A part product of an infinite
-// operand with a zero part is NaN where the f32 product is infinite, and a value
-// within half a bf16 step of the largest f32 rounds to an infinite part; this
-// gives such elements the f32 kernel's result (infinities, NaN and overflow).
-template <int MODE, int PRO, bool F16>
-__device__ float split_exact_dot(const GemmArgs &p, int row, int col, int k_begin, int k_end) {
-    const ConvRow r = MODE >= kConvAligned ? conv_row(p, row) : ConvRow{PRO == kProAffine ? row / p.pro_rows : 0, 0, 0, true};
-    float s = 0.0f;
+// One wave's sums on the f32 instructions, straight from memory: rows m.. of A, columns
+// n.. and the K values of wave group wk. For tiles with a sum that is infinite or NaN (a
+// part product of an infinite value with a zero part is NaN where the f32 product is
+// infinite, and a value within half a bf16 step of the largest f32 rounds to an infinite
+// part) or too small for its operands' bits (split_bf16.hpp). 2048x1280x1280 of nothing
+// but such values: 170 us against 62.
+template <int FM, int FN, int WK, int MODE, int PRO, bool F16>
+__device__ __forceinline__ void split_redo(const GemmArgs &p, int m, int n, int wk, int lane, floatx4 (&sum)[FM][FN]) {
+    const int l16 = lane & 15, kg = lane >> 4;
+    const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(p.a, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t a2_rsrc = make_rsrc(p.a2 ? p.a2 : p.a, p.a2 ? p.a2_bytes : p.a_bytes);
+    const __amdgpu_buffer_rsrc_t b_rsrc = make_rsrc(p.b, p.b_bytes);
+    ConvRow crow[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int row = m + 16 * i + l16;
+        if constexpr (MODE >= kConvAligned) crow[i] = conv_row(p, row);
+        else crow[i] = ConvRow{PRO == kProAffine ? min(row, p.M - 1) / p.pro_rows : 0, 0, 0, true};
+#pragma unroll
+        for (int j = 0; j < FN; ++j) sum[i][j] = zero4();
+    }
 #pragma nounroll
-    for (int k = k_begin; k < k_end; ++k) {
-        float a = 0.0f;
-        if constexpr (MODE == kDense) {
-            a = p.a2 && k >= p.ka ? p.a2[int64_t(row) * p.lda2 + (k - p.ka)] : p.a[int64_t(row) * p.lda + k];
-            if constexpr (PRO == kProAffine) {
-                const int64_t i = int64_t(r.b) * p.K + k;
-                a = __builtin_fmaf(a, p.psc[i], p.psh[i]);
-                if (p.psilu) a = ref_silu(a);
-            }
-        } else {
-            const int tap = k / p.ci, c = k - tap * p.ci;
-            const int64_t off = conv_src(p, r, tap / 3, tap % 3);
-            if (off >= 0) {
-                a = p.a[off + c];
-                if constexpr (PRO == kProAffine) a = prologue1(p, r.b, c, a);
+    for (int k0 = wk * kSK; k0 < p.K; k0 += WK * kSK) {
+        int tky = 0, tkx = 0, tci = 0;
+        if constexpr (MODE == kConvAligned) {
+            const int tap = k0 / p.ci;
+            tci = k0 - tap * p.ci;
+            tky = tap / 3;
+            tkx = tap - tky * 3;
+        }
+        const bool sec = MODE == kDense && p.a2 && k0 >= p.ka;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = k0 + 16 * h + 4 * kg;
+            floatx4 a[FM];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                a[i] = sec ? load_a_buf<MODE, PRO>(p, a2_rsrc, crow[i], m + 16 * i + l16, k - p.ka, p.K - p.ka, 0, 0, 0, p.lda2)
+                           : load_a_buf<MODE, PRO>(p, a_rsrc, crow[i], m + 16 * i + l16, k, p.K, tky, tkx, tci);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const floatx4 b = load_b_buf<F16>(p, b_rsrc, n + 16 * j + l16, k, p.K);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < FM; ++i) sum[i][j] = Mf<16>::mfma(a[i][t], b[t], sum[i][j]);
             }
         }
-        const int64_t e = int64_t(col) * p.ldb + k;
-        const float b = F16 ? float(static_cast<const _Float16 *>(p.b)[e]) : static_cast<const float *>(p.b)[e];
-        s = __builtin_fmaf(a, b, s);
-        if (s != s) break;  // NaN stays NaN
     }
-    return s;
 }
 
 // WM x WK waves: wave (wm, wk) owns rows [wm * TM, (wm + 1) * TM) of the tile,
@@ -333,27 +349,25 @@ __global__ __launch_bounds__(64 * WM * WK, WK <= 2 ? 4 : 2) void gemm_split_kern
 
     __shared__ float ln_st[PRO >= kProLn ? 2 * BM : 1];
     if constexpr (PRO == kProLnPart) ln_stats_from_parts<BM, NT>(p, m0, ln_st);
-    float probe = 0.0f;  // NaN once any sum is infinite or NaN
+    SplitProbe probe;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
+            for (int v = 0; v < 4; v += 2) {
                 acc[i][j][v] = acc[i][j][v] + low[i][j][v];
-                probe = __builtin_fmaf(acc[i][j][v], 0.0f, probe);
+                acc[i][j][v + 1] = acc[i][j][v + 1] + low[i][j][v + 1];
+                probe.see(acc[i][j][v], acc[i][j][v + 1]);
             }
-    auto mend = [&](float *tile) {
-        for (int e = tid; e < BM * BN; e += NT) {
-            const int rr = e / BN, cc = e - rr * BN;
-            if (m0 + rr >= p.M || n0 + cc >= p.N) continue;
-            float &v = tile[rr * L::CS + cc];
-            if (!(__builtin_fabsf(v) < __builtin_inff()))
-                v = split_exact_dot<MODE, PRO, F16>(p, m0 + rr, n0 + cc, 0, p.K);
-        }
+    auto redo = [&](floatx4 (&sum)[FM][FN]) {
+        // the lane's number again, so that nothing this derives from it is kept through the loop
+        int lane2 = lane;
+        asm volatile("" : "+v"(lane2));
+        split_redo<FM, FN, WK, MODE, PRO, F16>(p, m0 + wm * TM, n0, wk, lane2, sum);
     };
     write_tile<BM, BN, WM, 1, WK, 16, EPI, false>(p, smem, acc, m0, n0, 0, PRO >= kProLn ? ln_st : nullptr,
-                                                  probe != probe, mend);
+                                                  probe.bad(), redo);
 }
 
 // The tilings: rows per wave, columns, waves over the rows, wave groups over K;

@@ -70,16 +70,15 @@ __device__ __forceinline__ void split_pair(float a, float b, int e, const SplitS
 
 // Whether any of the sums seen is infinite, NaN, or too small for its operands' bits.
 struct SplitProbe {
-    float sick = 0.0f;             // NaN once a sum is infinite or NaN
+    float most = 0.0f;             // the largest magnitude, NaN once a sum is NaN
     uint32_t least = 0xffffffffu;  // the smallest 2 * |bits| - 1: a zero counts as the largest
-    __device__ __forceinline__ void see(float s) {
-        sick = __builtin_fmaf(s, 0.0f, sick);
-        const uint32_t b = (__builtin_bit_cast(uint32_t, s) << 1) - 1;
-        least = b < least ? b : least;
+    __device__ __forceinline__ void see(float a, float b) {
+        most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)), most);
+        least = min(least, min((__builtin_bit_cast(uint32_t, a) << 1) - 1, (__builtin_bit_cast(uint32_t, b) << 1) - 1));
     }
     __device__ __forceinline__ bool bad() const {
         constexpr uint32_t kLeast = (127u - 72u) << 24;  // 2^-72
-        return sick != sick || least < kLeast - 1;
+        return !(most < __builtin_inff()) || least < kLeast - 1;
     }
 };
 

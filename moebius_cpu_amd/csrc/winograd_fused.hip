@@ -410,7 +410,7 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
                 for (int kk = 0; kk < 4; ++kk) {
                     if constexpr (!F32) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) probe.see(y[kk][e]);
+                        for (int e = 0; e < 4; e += 2) probe.see(y[kk][e], y[kk][e + 1]);
                     }
                     y[kk] = add4(y[kk], bv);
                 }
