@@ -397,12 +397,19 @@ struct SplitPlan {
 // 10%). The sum over the UNet's GEMMs comes within 0.5% of the best choice for each.
 // Kept by the f32 kernels: under 0.8 GFLOP, where fixed costs decide (4096x256x128
 // 7.5 against 6.5 us, 64x1280x1280 11.1 against 10.4), and small grids of long K,
-// which they split over workgroups (256x640x5760 44 against 35 us). A few rows of a
-// large weight (the time projections, 2x11200x1280: 20 against 25 us) are bound by
-// reading it and take the small tile. Convs leave 64x80 with two wave groups out: the
+// which they split over workgroups (256x640x5760 44 against 35 us). Up to 32 rows of a
+// large weight (the time projections) are bound by reading it: the narrowest tile
+// whose columns are one round of the CUs, over weights not yet in the caches: 2x8192x1024
+// 11.9 us (32 columns) against 13.4, 2x11200x1280 15.2 (48) against 17.8, 32x16384x1280
+// 20.9 (64) against 23.5, 2x20480x1280 21.6 (80) against 26.5, 16x1280x11520 64 against
+// 84; not past that round (2x25600x1280 34 against 31) or under K = 768 (32x16384x512
+// 11.6 against 11.2), and not the convs, whose K the f32 kernels split over workgroups
+// (an 8x8 map's stride 2, 16x1280x11520: 78 against 54 us). Convs leave 64x80 with two wave groups out: the
 // gather's addresses spill there (64x64 x 320 channels 86 us, 64x48 69, f32 80).
 inline SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int cus, int batch, bool conv) {
-    if (M <= 32 && N * K >= (int64_t(1) << 23) && batch == 1) return SplitPlan{16, 48, 2, 4};
+    if (M <= 32 && K >= 768 && N * K >= (int64_t(1) << 23) && batch == 1 && !conv)
+        for (const int bn : {32, 48, 64, 80})
+            if (ceil_div(N, int64_t(bn)) <= cus) return SplitPlan{16, bn, 2, 4};
     const double products = double(M) * double(N) * double(K) * batch;
     if (products < 4e8) return SplitPlan{};
     SplitPlan best;
