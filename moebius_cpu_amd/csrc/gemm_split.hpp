@@ -409,29 +409,36 @@ struct SplitPlan {
 // 11.6 against 11.2), and not the convs, whose K the f32 kernels split over workgroups
 // (an 8x8 map's stride 2, 16x1280x11520: 78 against 54 us). Convs leave 64x80 with two wave groups out: the
 // gather's addresses spill there (64x64 x 320 channels 86 us, 64x48 69, f32 80).
-inline SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int cus, int batch, bool conv) {
+// gn_rows: the rows per item where the output's GroupNorm partials are wanted (0: not);
+// a tile height that does not divide them costs the next GroupNorm a statistics launch
+// (priced, 1568x512x512 and the GroupNorm's fold take 17.5 us for 19.6, 2592 rows 23.0 for
+// 24.3, 3136 26.7 for 26.6).
+inline SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int cus, int batch, bool conv, int gn_rows) {
     if (M <= 32 && K >= 768 && N * K >= (int64_t(1) << 23) && batch == 1 && !conv)
         for (const int bn : {32, 48, 64, 80})
             if (ceil_div(N, int64_t(bn)) <= cus) return SplitPlan{16, bn, 2, 4};
     const double products = double(M) * double(N) * double(K) * batch;
     if (products < 4e8) return SplitPlan{};
+    // the statistics launch of a tiling whose rows would straddle items
+    auto stats = [&](int64_t rows) { return gn_rows && gn_rows % rows ? 5.0 + double(M * N) * 4.0 / 4.5e6 : 0.0; };
     SplitPlan best;
-    double cost = (11.5 + products * (2.0 / 116e6)) * (K < 256 ? 0.97 : 1.0);
+    double cost = (11.5 + products * (2.0 / 116e6)) * (K < 256 ? 0.97 : 1.0) + stats(32);
     for (const SplitTile &t : kSplitTiles) {
         if (conv && t.bn == 80 && t.wk == 2) continue;
         const int64_t tiles = ceil_div(M, int64_t(t.tm) * t.wm) * ceil_div(N, int64_t(t.bn)) * batch;
-        const double c = t.launch + double(ceil_div(tiles, int64_t(cus))) * (t.round + t.per_k * 1e-3 * double(K));
+        const double c = t.launch + double(ceil_div(tiles, int64_t(cus))) * (t.round + t.per_k * 1e-3 * double(K)) +
+                         stats(t.tm * t.wm);
         if (c < cost) best = SplitPlan{t.tm, t.bn, t.wm, t.wk}, cost = c;
     }
     return best;
 }
 
 // The same under the context's tuning (gemm_split; gemm_plan forces an f32 tiling).
-inline SplitPlan split_plan_for(const Context &ctx, int64_t M, int N, int K, int batch, bool conv) {
+inline SplitPlan split_plan_for(const Context &ctx, int64_t M, int N, int K, int batch, bool conv, int gn_rows = 0) {
     ShapePlan forced;
     if (!ctx.tune.gemm_split || K % 4 || forced_plan(ctx.tune, int(M), N, K, forced)) return SplitPlan{};
     if (ctx.tune.split_tm) return SplitPlan{ctx.tune.split_tm, ctx.tune.split_bn, ctx.tune.split_wm, ctx.tune.split_wk};
-    return plan_split(M, N, K, ctx.cu_count, batch, conv);
+    return plan_split(M, N, K, ctx.cu_count, batch, conv, gn_rows);
 }
 
 template <int TM, int BN, int WM, int WK, int MODE, int PRO, bool F16>
@@ -478,7 +485,7 @@ bool launch_split_tile(Context &ctx, GemmArgs &p, const SplitPlan &s, GemmEpilog
 // A vector A operand (checked by the caller) and vector weight rows.
 template <int MODE, int PRO>
 bool launch_split(Context &ctx, GemmArgs &p, WeightType wt, GemmEpilogue epi, int batch) {
-    const SplitPlan s = split_plan_for(ctx, p.M, p.N, p.K, batch, MODE >= kConvAligned);
+    const SplitPlan s = split_plan_for(ctx, p.M, p.N, p.K, batch, MODE >= kConvAligned, p.gnp ? p.gn_item_rows : 0);
     const int esz = wt == kF16 ? 2 : 4;
     if (!s.tm || p.ldb % 4 || reinterpret_cast<uintptr_t>(p.b) % (4 * esz) || (batch > 1 && p.b_bs % 4)) return false;
     return wt == kF16 ? launch_split_tile<0, MODE, PRO, true>(ctx, p, s, epi, batch)

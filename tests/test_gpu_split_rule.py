@@ -2,6 +2,8 @@
 its rule, read from the launch timing's configuration; and the results either way."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,22 @@ def test_few_pixels(ctx, tune, h, w, ci, co, stride):
     assert config.startswith("f32 ") and "split" not in config
     tune("gemm_split", "16,32,2,4")
     assert close(got, run(ctx, tune, conv, x)[0], 9 * ci)
+
+
+# rows per item that 128, or 64 and 128, do not divide: the taller tiles are faster but for the
+# statistics launch that the next GroupNorm would need
+@pytest.mark.parametrize("h,w", [(56, 56), (51, 64), (32, 49), (64, 64)])
+def test_group_norm_partials_are_kept(ctx, h, w):
+    c = 512
+    rng = np.random.default_rng(h)
+    x = rng.standard_normal((1, h, w, c), dtype=np.float32)
+    wt = E.Param(ctx, rng.standard_normal((c, c), dtype=np.float32) / np.float32(np.sqrt(c)))
+    out, part = E.DeviceArray(ctx, (1, h, w, c)), E.DeviceArray(ctx, (-(-h * w // 32), c, 2))
+    xd, rows = E.DeviceArray.from_numpy(ctx, x), ctypes.c_uint32()
+    E.check(E.lib().mh_conv1x1_gn_partials(ctx.h, xd.ptr, 1, h, w, c, wt.ptr, wt.dtype, c, None, None, out.ptr, part.ptr,
+                                           ctypes.byref(rows)))
+    assert rows.value > 0 and h * w % rows.value == 0
+    y = out.numpy().reshape(-1, c).astype(np.float64)
+    sums = part.numpy()[:h * w // rows.value].astype(np.float64).sum(axis=0)
+    # 32 to 128 values a partial, summed in f32
+    assert np.abs(sums[:, 1] - (y * y).sum(axis=0)).max() <= 128 * 2.0 ** -24 * (y * y).sum(axis=0).max()
