@@ -119,15 +119,18 @@ bool set_tuning(Tuning &t, const char *key, const char *value) {
     if (k == "taps_r16") return to_int(t.taps_r16, 0) && t.taps_r16 >= 0 && t.taps_r16 <= 1;
     if (k == "wino_u16") return to_int(t.wino_u16, 1) && t.wino_u16 >= 0 && t.wino_u16 <= 1;
     if (k == "wino_v16") return to_int(t.wino_v16, 1) && t.wino_v16 >= 0 && t.wino_v16 <= 1;
-    if (k == "gemm_split") {  // "0", "1" or "tm,bn,wm,wk"
+    if (k == "gemm_split") {  // "0", "1" or "tm,bn,wm,wk" of a tiling that there is
         t.split_tm = t.split_bn = t.split_wm = t.split_wk = 0;
         t.gemm_split = 1;
-        int tm = 0, bn = 0, wm = 0, wk = 0;
-        if (std::sscanf(v.c_str(), "%d,%d,%d,%d", &tm, &bn, &wm, &wk) == 4) {
+        int tm = 0, bn = 0, wm = 0, wk = 0, end = 0, on = 1;
+        if (std::sscanf(v.c_str(), "%d,%d,%d,%d%n", &tm, &bn, &wm, &wk, &end) == 4) {
+            if (v[size_t(end)] || !split_tiling_exists(tm, bn, wm, wk)) return false;
             t.split_tm = tm, t.split_bn = bn, t.split_wm = wm, t.split_wk = wk;
             return true;
         }
-        return to_int(t.gemm_split, 1) && t.gemm_split >= 0 && t.gemm_split <= 1;
+        if (!to_int(on, 1) || on < 0 || on > 1) return false;
+        t.gemm_split = on;
+        return true;
     }
     if (k == "dw_out16") return to_int(t.dw_out16, 1) && t.dw_out16 >= 0 && t.dw_out16 <= 1;
     if (k == "tap_jq") return to_int(t.tap_jq, 1) && (t.tap_jq == 1 || t.tap_jq == 2);

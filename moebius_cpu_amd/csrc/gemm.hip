@@ -85,6 +85,12 @@ bool exact_reads_widened(const Context &ctx, int64_t rows, int n, int k, bool co
     return ctx.precision == Precision::Exact && !split_plan_for(ctx, rows, n, k, 1, conv).tm;
 }
 
+bool split_tiling_exists(int tm, int bn, int wm, int wk) {
+    for (const SplitTile &t : kSplitTiles)
+        if (t.tm == tm && t.bn == bn && t.wm == wm && t.wk == wk) return true;
+    return false;
+}
+
 void conv1x1(Context &ctx, const float *x, int64_t pixels, int c_in, const void *weight, WeightType wt, int c_out,
              const float *bias, const float *residual, float *out, GemmEpilogue epi, const ResidualAffine *raff,
              const float *residual2, GnPartials *gn, const ResidualAffine *x_aff, const float *x2, int c2,

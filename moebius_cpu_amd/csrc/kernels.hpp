@@ -46,6 +46,9 @@ void tile_items(Context &ctx, const float *src, int64_t item, int n, float *dst)
 // bf16 kernels prefer the f16 values. Either copy gives the same bits.
 bool exact_reads_widened(const Context &ctx, int64_t rows, int n, int k, bool conv);
 
+// Whether the split bf16 kernels have this tiling (gemm_split.hpp).
+bool split_tiling_exists(int tm, int bn, int wm, int wk);
+
 // ---- normalisation (norm.hip) ----
 // add (optional): per item and channel, item b's row at add + b * add_ld (add_ld 0: c).
 // x2 (optional): the input is [x | x2] per pixel, x holding the first c - c2

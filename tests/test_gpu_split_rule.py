@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from moebius_cpu_amd import engine as E
+from tests.test_gpu_split import TILES
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +86,32 @@ def test_group_norm_partials_are_kept(ctx, h, w):
     sums = part.numpy()[:h * w // rows.value].astype(np.float64).sum(axis=0)
     # 32 to 128 values a partial, summed in f32
     assert np.abs(sums[:, 1] - (y * y).sum(axis=0)).max() <= 128 * 2.0 ** -24 * (y * y).sum(axis=0).max()
+
+
+# the forced tilings of the split kernel's tests are the ones that run, and the planner's choice at a
+# shape above its line is one of them
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("f16", [False, True])
+def test_the_tiling_that_runs(ctx, tune, tile, f16):
+    rng = np.random.default_rng(5)
+    tune("gemm_split", tile)
+    px, ci, co = ((64, 64), 320, 320) if tile == "1" else ((9, 11), 64, 70)
+    x = rng.standard_normal((1, *px, ci), dtype=np.float32)
+    dense = E.Conv1x1(ctx, ci, co, E.Param(ctx, rng.standard_normal((co, ci)).astype(np.float16 if f16 else np.float32),
+                                           f16=f16))
+    conv = E.Conv3x3(ctx, ci, co, E.Param(ctx, rng.standard_normal((co, 3, 3, ci)).astype(np.float16 if f16 else np.float32),
+                                          f16=f16))
+    for op in (dense, conv):
+        config = run(ctx, tune, op, x)[1]
+        if tile == "1":
+            assert config.startswith("f32 split ")
+        else:
+            tm, bn, wm, wk = (int(v) for v in tile.split(","))
+            assert config.startswith(f"f32 split {tm * wm}x{bn} waves {wm}x1x{wk}")
+
+
+@pytest.mark.parametrize("value", ["16,80,8", "16,80,8,1,1", "16,80,8,1 ", "16,96,8,1", "32,80,4,1", "2", "-1", "x"])
+def test_an_unknown_tiling_is_refused(ctx, value):
+    with pytest.raises(E.MoebiusError):
+        ctx.set_tuning("gemm_split", value)
+    ctx.set_tuning("gemm_split", None)
