@@ -68,12 +68,17 @@ __device__ __forceinline__ void split_pair(float a, float b, int e, const SplitS
     s.q[2].p[e] = round_pair(a, b);
 }
 
+// The larger magnitude, NaN if either is NaN.
+__device__ __forceinline__ float abs_max(float a, float b) {
+    return __builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b));
+}
+
 // Whether any of the sums seen is infinite, NaN, or too small for its operands' bits.
 struct SplitProbe {
     float most = 0.0f;             // the largest magnitude, NaN once a sum is NaN
     uint32_t least = 0xffffffffu;  // the smallest 2 * |bits| - 1: a zero counts as the largest
     __device__ __forceinline__ void see(float a, float b) {
-        most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)), most);
+        most = abs_max(abs_max(a, b), most);
         least = min(least, min((__builtin_bit_cast(uint32_t, a) << 1) - 1, (__builtin_bit_cast(uint32_t, b) << 1) - 1));
     }
     __device__ __forceinline__ bool bad() const {

@@ -405,16 +405,20 @@ __global__ __launch_bounds__(kFThreads, 2) void wino_fused_kernel(FArgs a) {
                 y[1] = add4(add4(m1[0], m1[1]), m1[2]);
                 y[2] = sub4(sub4(m0[1], m0[2]), m0[3]);
                 y[3] = sub4(sub4(m1[1], m1[2]), m1[3]);
-                SplitProbe probe;  // every plane is in one of the four
+                if constexpr (!F32) {
+                    // The largest of the tile's four pixels in each channel: every plane is in
+                    // one of them, and a small one beside it is a difference of its terms.
+                    float top[4];
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    if constexpr (!F32) {
-#pragma unroll
-                        for (int e = 0; e < 4; e += 2) probe.see(y[kk][e], y[kk][e + 1]);
-                    }
-                    y[kk] = add4(y[kk], bv);
+                    for (int e = 0; e < 4; ++e)
+                        top[e] = abs_max(abs_max(y[0][e], y[1][e]), abs_max(y[2][e], y[3][e]));
+                    SplitProbe probe;
+                    probe.see(top[0], top[1]);
+                    probe.see(top[2], top[3]);
+                    sick = sick || probe.bad();
                 }
-                sick = sick || probe.bad();
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) y[kk] = add4(y[kk], bv);
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) {
                     const int oy = 2 * ty + (kk >> 1), ox = 2 * tx + (kk & 1);
