@@ -1258,7 +1258,8 @@ inline Plan plan_for(int M, int N, int K, int cus, bool dense) {
 }
 
 // Wide-layout plan for a dense GEMM with vector f32 weights, or bm = 0 to keep
-// plan_for's. Timed inside the UNet step (kernel trace of a whole step, each
+// plan_for's: for f32 products throughout (tuning gemm_split 0), since plan_split takes
+// these shapes unless K is under about 60. Timed inside the UNet step (kernel trace of a whole step, each
 // GEMM in its place: cold weights, its producer's output just written back),
 // which is not what a GEMM repeated on its own operands measures: of the
 // layouts that beat the square tilings alone, these two also win in the step:

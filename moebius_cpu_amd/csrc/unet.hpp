@@ -28,7 +28,10 @@ struct NamedTensor {
 // after widening each value as they load it, without the conversion in the loop and
 // with the f32 kernels' tilings. The split kernels read the f16 copy: half the bytes,
 // and a value of two bf16 parts makes five part products of six, the sixth being
-// zero, so the sums are the same bits (UNet step with CFG 6.33 -> 5.98 ms).
+// zero, so the sums are the same bits (UNet step with CFG 6.33 -> 5.98 ms). Every f16
+// weight keeps its widening (0.9 GB for the UNet), since a GEMM's kernel depends on its
+// rows and the tuning: with the defaults those under 0.8 GFLOP read it, and long K on
+// small grids.
 struct DParam {
     const void *p = nullptr;
     WeightType wt = kF32;

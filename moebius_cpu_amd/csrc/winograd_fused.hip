@@ -18,17 +18,17 @@
 // wino_output_kernel) to one tile and four channels, adding bias and the optional
 // residual.
 //
-// What bounds it (MI355X, 512x512x128 -> 128, parts taken out of a copy): the
-// products alone 130 us, with the transforms 148, with the patch and U loads 221,
-// with the output transform and its stores 279; on the f32 instructions the same
-// conv took 358 us, its products alone 239. The loads cost what they do because
+// What bounds it (MI355X, 512x512x128 -> 128, parts taken out of a copy, all on one
+// board): the products alone 130 us, with the transforms 148, with the patch and U
+// loads 221, with the output transform and its stores 279 (257 for a whole call on
+// others); on the f32 instructions the same conv took 358 us, its products alone 239. The loads cost what they do because
 // the vector L1 serves 96 KB of U and 64 KB of patches per chunk and workgroup:
 // 64 tiles per workgroup, twice what the f32 kernel took, halve U's share, and
 // 128 accumulators per lane are what that leaves room for. The registers are full:
 // a few more live values spill the patch in the loop (392 us), so the output
 // transform's numbers are derived anew from the thread's, the patch's validity is
 // kept in scalar masks and the next item's loads wait for the sums to leave.
-// 128x128x512 -> 512: 402 us in f32, 251 here. VAE decode 12.97 -> 9.77 ms.
+// 128x128x512 -> 512: 402 us in f32, 230 to 251 here. VAE decode 12.97 -> 9.77 ms.
 #include <algorithm>
 
 #include "common.hpp"
@@ -489,10 +489,11 @@ void launch_fused(Context &ctx, const FArgs &a) {
 // per CU, 3.6 us for each 16 input channels and 6 for the output transform, 8 for
 // the two launches, and the weights' reordering where the caller has no copy. The
 // three: V and M of 16 planes at 4 TB/s, the products, 12 for the launches. A round
-// that is nearly empty costs as much as a full one, so the line is no tile count:
-// 2x64x64x512 fills one round (150 -> 125 us) and one 64x64x512 half of it (83
-// against 125); 108x148x256 97 -> 71 us; 512x512x128 takes 8 rounds and 251 us
-// against 480, 128x128x512 2 and 251 against 300. Up to the measured 512 channels.
+// that is nearly empty costs as much as a full one, so the line is no tile count.
+// Whole calls, the weights reordered in them, three kernels -> one: 2x64x64x512, one
+// round, 137 -> 124 us; 64x64x512, half a round, 76 -> 115; 108x148x256 89 -> 66;
+// 512x512x128, 8 rounds, 580 -> 257; 128x128x512, 2 rounds, 276 -> 230; 130x130x512,
+// one workgroup past 2 rounds, 290 -> 319. Up to the measured 512 channels.
 bool fused_is_faster(int64_t tiles, int c_in, int c_out, int cus, bool have_uf) {
     if (c_in > 512 || c_out > 512) return false;
     const int64_t items = ceil_div(tiles, kFT) * (c_out / kFC);

@@ -1,5 +1,5 @@
 """The Winograd F(2x2,3x3) conv in one kernel (winograd_fused.hip: input
-transform, the 16 plane products and the output transform of a 32-tile x
+transform, the 16 plane products and the output transform of a 64-tile x
 64-channel block kept on chip) against the oracle's conv (src/engine/
 winograd.rs:48-120) at the f32 bar and against the three-kernel path
 (transforms + batched GEMM; tuning "wino_fused" 0): odd sizes with partial
