@@ -16,8 +16,10 @@
 // absolute sums of its two operands' K values over s, under 2^-26 while s is at least
 // 2^-72 and those sums below 2^36. So the kernels take a sum that is smaller and not
 // zero, as one that is infinite or NaN, for one to be redone on the f32 instructions
-// (SplitProbe). Scaling every operand by 2^16 before it is split keeps all bits without
-// that, and cost 1 to 3% (UNet step with CFG 6.21 -> 6.40 ms).
+// (SplitProbe). A sum that is zero because all its operands round to zero (under 2^-134)
+// stays zero; with the other side's absolute sum below 2^36 it is under 2^-98. Scaling
+// every operand by 2^16 before it is split keeps all bits without that, and cost 1 to
+// 3% (UNet step with CFG 6.21 -> 6.40 ms).
 #pragma once
 
 #include <hip/hip_runtime.h>
